@@ -501,14 +501,14 @@ extern "C" int slc_hip_prefill_attention_classes(
                        (tokens + 15) / 16 <= 65535 &&
                        (tokens + kQueries - 1) / kQueries <= 65535;  // grid z: query blocks
   // The grouped kernel: GQA groups of 1, 2, 4, 7 or 8 heads, and a mask (if
-  // any) with unit key stride and 16-byte aligned rows.
+  // any) whose [T, T] plane spans less than 2^31 bytes, in any row order
+  // (16-byte chunks where its rows allow, elements otherwise).
   const bool group_ok = groups == 1 || groups == 2 || groups == 4 || groups == 7 || groups == 8;
   const int64_t me = mask == nullptr ? 0 : slc_host::dtype_size(mask_dtype);
   const bool mask_ok =
       mask == nullptr ||
-      (m_sk == 1 && (m_sq * me) % 16 == 0 && (m_sb * me) % 16 == 0 &&
-       (reinterpret_cast<uintptr_t>(mask) & 15) == 0 &&
-       ((tokens - 1) * m_sq + tokens) * me < (1LL << 31));
+      (m_sk >= 1 && m_sq >= 0 && m_sk < (1LL << 31) / tokens && m_sq < (1LL << 31) / tokens &&
+       ((tokens - 1) * (m_sq + m_sk) + 1) * me < (1LL << 31));
   const bool out_ok = (reinterpret_cast<uintptr_t>(output) & 7) == 0 &&
                       ((o_sb | o_sh | o_st) & 3) == 0;
   // The grouped kernel takes the row max before the scale factor: positive

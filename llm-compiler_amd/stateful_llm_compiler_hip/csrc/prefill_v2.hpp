@@ -157,7 +157,8 @@ __global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attenti
     const void* __restrict__ mask, T* __restrict__ output, int tokens, int kv_heads,
     int64_t q_sb, int64_t q_sh, int64_t q_st, int64_t k_sb, int64_t k_sh, int64_t k_st,
     int64_t v_sb, int64_t v_sh, int64_t v_st, int64_t m_sb, int64_t m_sq, int64_t o_sb,
-    int64_t o_sh, int64_t o_st, float scale, const unsigned char* __restrict__ tile_class) {
+    int64_t o_sh, int64_t o_st, float scale, const unsigned char* __restrict__ tile_class,
+    int m_step) {
   using M = Mfma<T>;
   constexpr int kQB = QB;                // query blocks of 16 per consumer wave
   constexpr int kV2Queries = 16 * QB;    // queries per workgroup
@@ -228,6 +229,50 @@ __global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attenti
     const char* mbase = MK == 0 ? nullptr
                                 : static_cast<const char*>(mask) + (b * m_sb + static_cast<int64_t>(q0) * m_sq) * ME;
     const int q_rows = min(kV2Queries, tokens - q0);
+    // m_step != 0: mask rows that 16-byte loads cannot take (an odd number of
+    // tokens, a key stride other than 1): element loads into registers, then
+    // LDS writes to the places the direct loads would fill.  Only tiles whose
+    // mask is applied from memory (class 2) come here, a few per query block
+    // of a padded or ragged batch, so the one producer wave keeps up: B3 T839
+    // exact with a padded fp32 mask 5075 us on the wave-per-query kernel these
+    // shapes took before, 39 us here (T840, direct loads: 36 us); B2 T2047
+    // fp16 online 386 us (single-head kernel) -> 51 us (T2048: 46 us).
+    auto stage_mask = [&](unsigned char* dst, int k0, int keys) {
+      const __amdgpu_buffer_rsrc_t rm =
+          make_rsrc(mbase + static_cast<int64_t>(k0) * m_step * ME,
+                    ((static_cast<int64_t>(q_rows) - 1) * m_sq +
+                     static_cast<int64_t>(keys - 1) * m_step + 1) * ME);
+      // Offset of (row, key), or one past any range (reads zero) outside the tile.
+      auto offset = [&](int row, int key) {
+        return row < q_rows && key < keys ? static_cast<int>((row * m_sq + key * m_step) * ME) : -1;
+      };
+      constexpr int kRows = ME == 4 ? 1 : 2;  // rows per round: 64 lanes, one dword each
+      constexpr int kBatch = 8;               // rounds of loads in flight
+      const int r0 = ME == 4 ? 0 : lane >> 5;
+      const int dword = ME == 4 ? lane : lane & 31;  // dword of the tile row
+#pragma unroll 1
+      for (int base = 0; base < kV2Queries; base += kBatch * kRows) {
+        uint32_t w[kBatch];
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+          const int row = base + i * kRows + r0;
+          if constexpr (ME == 4) {
+            w[i] = static_cast<uint32_t>(
+                __builtin_amdgcn_raw_buffer_load_b32(rm, offset(row, dword), 0, 0));
+          } else {
+            const uint16_t lo = __builtin_amdgcn_raw_buffer_load_b16(rm, offset(row, 2 * dword), 0, 0);
+            const uint16_t hi = __builtin_amdgcn_raw_buffer_load_b16(rm, offset(row, 2 * dword + 1), 0, 0);
+            w[i] = lo | (static_cast<uint32_t>(hi) << 16);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i) {
+          const int row = base + i * kRows + r0;
+          *reinterpret_cast<uint32_t*>(dst + row * kMaskRow + (((dword >> 2) ^ (row & 7)) << 4) +
+                                       (dword & 3) * 4) = w[i];
+        }
+      }
+    };
     // Lane L of DMA instruction n fills LDS row 8n + L/8, chunk position L%8,
     // with the global 16-byte chunk (L%8) ^ (row & 7) of that row.
     auto issue = [&](int step, int stage) {
@@ -251,6 +296,10 @@ __global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attenti
         lds_dma16(rv, dst + kV2TileBytes + n * 1024, static_cast<int>(row * v_st * 2 + chunk * 16));
       }
       if constexpr (MK != 0) {
+        if (m_step != 0) {
+          if (want_mask && q_rows > 0) stage_mask(dst + 2 * kV2TileBytes, k0, rows);
+          return;
+        }
         // Mask rows are queries, chunks 8 keys; whole rows stay inside the
         // [T, T] plane (keys past T are masked as invalid anyway).
         const int64_t bytes = want_mask && q_rows > 0
@@ -571,6 +620,17 @@ __global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attenti
   }
 }
 
+// 0 where whole 16-byte mask chunks can be loaded (unit key stride, rows that
+// start on 16 bytes and end on a dword: a buffer range that ends inside a
+// dword reads that dword as zero, which would drop the last key of the last
+// row), else the key stride in elements for element loads.
+inline int mask_step(const void* mask, const int64_t* st, int tokens, int es) {
+  const bool chunks = st[11] == 1 && (st[10] * es) % 16 == 0 && (st[9] * es) % 16 == 0 &&
+                      (static_cast<int64_t>(tokens) * es) % 4 == 0 &&
+                      (reinterpret_cast<uintptr_t>(mask) & 15) == 0;
+  return chunks ? 0 : static_cast<int>(st[11]);
+}
+
 template <typename T, int G, int MK, bool CAUSAL, int QB>
 int launch_v2(const void* q, const void* k, const void* v, const void* mask, void* out,
               int64_t batch, int tokens, int kv_heads, const int64_t* st, float scale,
@@ -587,7 +647,8 @@ int launch_v2(const void* q, const void* k, const void* v, const void* mask, voi
                      stream, static_cast<const T*>(q), static_cast<const T*>(k),
                      static_cast<const T*>(v), mask, static_cast<T*>(out), tokens, kv_heads,
                      st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7], st[8], st[9], st[10],
-                     st[12], st[13], st[14], scale, MK != 0 ? classes : nullptr);
+                     st[12], st[13], st[14], scale, MK != 0 ? classes : nullptr,
+                     MK != 0 ? mask_step(mask, st, tokens, mask_elem_bytes<MK>()) : 0);
   return slc_host::check_launch("slc_hip_prefill_attention(grouped)");
 }
 

@@ -628,3 +628,54 @@ def test_prefill_short_and_long_workgroups_agree(gpu, kind):
     torch.cuda.synchronize()
     assert torch.isfinite(short_form.float()).all()
     assert torch.equal(long_form[:8].view(torch.int16), short_form.view(torch.int16))
+
+
+@pytest.mark.parametrize("tokens,layout", [(17, "rows"), (65, "rows"), (130, "rows"), (500, "rows"), (839, "rows"),
+                                           (96, "offset"), (97, "strided"), (64, "shared"), (131, "transposed")])
+@pytest.mark.parametrize("order", ["online", "exact"])
+@pytest.mark.parametrize("mask_dtype", [torch.float32, torch.bfloat16])
+def test_prefill_masks_in_any_layout_agree(gpu, tokens, layout, order, mask_dtype):
+    """A mask whose rows 16-byte loads cannot take (an odd row length, a start
+    off the 16-byte grid, a key stride above 1, one plane or one row shared)
+    gives bit for bit what the same values in aligned rows give, and stays
+    within the bf16 bar of the oracle."""
+
+    from stateful_llm_compiler_hip.backends import hip_prefill_attention
+
+    announce(f"prefill mask layout={layout} {mask_dtype} T={tokens} order={order}")
+    batch = 3
+    g = generator(tokens)
+    q = torch.randn(batch, 14, tokens, 64, generator=g).bfloat16()
+    k = torch.randn(batch, 2, tokens, 64, generator=g).bfloat16()
+    v = torch.randn(batch, 2, tokens, 64, generator=g).bfloat16()
+    pad = torch.randint(0, tokens // 3 + 1, (batch, 1, 1), generator=g)
+    at = torch.arange(tokens)
+    hidden = (at.view(1, 1, -1) > at.view(1, -1, 1)) | (
+        (at.view(1, 1, -1) < pad) & (at.view(1, 1, -1) != at.view(1, -1, 1)))
+    values = torch.randn(batch, tokens, tokens, generator=g).masked_fill(hidden, float("-inf"))
+    values = values.unsqueeze(1).to(mask_dtype)
+    if layout == "shared":  # one plane for the whole batch, one finite row for every query
+        values = values[:1, :, -1:].expand(batch, 1, tokens, tokens)
+        values = torch.where(torch.isinf(values), torch.zeros_like(values), values)
+    es = values.element_size()
+    rows = -(-tokens // 16) * 16
+    aligned = torch.zeros(batch, 1, tokens, rows, dtype=mask_dtype, device=gpu)[..., :tokens]
+    aligned.copy_(values)
+    if layout == "rows":
+        odd = values.to(gpu).contiguous()
+    elif layout == "offset":
+        odd = torch.empty(values.numel() + 1, dtype=mask_dtype, device=gpu)[1:].view(values.shape).copy_(values)
+    elif layout == "strided":
+        odd = torch.empty(batch, 1, tokens, 2 * tokens + 1, dtype=mask_dtype, device=gpu)[..., 1::2].copy_(values)
+    elif layout == "transposed":
+        odd = values.transpose(2, 3).contiguous().to(gpu).transpose(2, 3)
+    else:
+        odd = torch.empty(1 + tokens, dtype=mask_dtype, device=gpu)[1:].copy_(values[0, 0, 0])
+        odd = odd.view(1, 1, 1, tokens).expand(batch, 1, tokens, tokens)
+    assert torch.equal(odd.cpu(), values) and (aligned.stride(2) * es) % 16 == 0
+    args = (q.to(gpu), k.to(gpu), v.to(gpu))
+    wanted = hip_prefill_attention(*args, aligned, scale=0.125, softmax_order=order)
+    actual = hip_prefill_attention(*args, odd, scale=0.125, softmax_order=order)
+    torch.cuda.synchronize()
+    assert torch.equal(actual.view(torch.int16), wanted.view(torch.int16))
+    assert_bf16_close(actual.cpu(), ref.prefill_attention(q, k, v, values, groups=7, scale=0.125, causal=False))
