@@ -170,6 +170,10 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 int gemm_residual(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                   const void* w, const void* bias, const void* residual, int64_t r_rs, void* y,
                   int64_t y_rs, int dtype, hipStream_t stream);
+// fp32 linear on the fp32 matrix cores (linear_f32.hip); SLC_ERR_UNSUPPORTED
+// (nothing launched) for shapes its kernels do not take.
+int linear_f32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
+               int64_t x_rs, int64_t y_rs, hipStream_t stream);
 bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                           int dtype);
 int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,

@@ -17,8 +17,8 @@
 //  * Decode-sized M (<= 64) takes a dedicated weight-streaming kernel (split-K
 //    across the waves of a workgroup, see linear_skinny_kernel); prefill-sized
 //    M uses 128 x 128 tiles (MFMA-bound).
-// fp32 (and shapes the vector path cannot take) use a classic LDS-tiled
-// FMA kernel.
+// fp32 runs on the fp32 matrix cores (linear_f32.hip); shapes neither vector
+// path can take use a classic LDS-tiled FMA kernel.
 #include <type_traits>
 
 #include "common.hpp"
@@ -978,7 +978,7 @@ int launch_skinny(const void* x, const void* w, const void* bias, void* y, int M
   return slc_host::check_launch("slc_hip_linear(skinny)");
 }
 
-// Classic 16 x 16 LDS-tiled FMA GEMM for fp32 and unaligned shapes.
+// Classic 16 x 16 LDS-tiled FMA GEMM for unaligned shapes.
 template <typename T>
 __global__ __launch_bounds__(256) void linear_generic_kernel(
     const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias,
@@ -1372,6 +1372,12 @@ extern "C" int slc_hip_linear_tile(const void* input, const void* weight,
   if (vec_ok && dtype == SLC_F16)
     return dispatch_mfma<slc::f16_t>(input, weight, bias, output, M, N, K,
                                      in_stride_row, out_stride_row, s, tile);
+  if (dtype == SLC_F32) {
+    const int rc = slc_host::linear_f32(static_cast<const float*>(input), static_cast<const float*>(weight),
+                                        static_cast<const float*>(bias), static_cast<float*>(output), M,
+                                        N, K, in_stride_row, out_stride_row, s);
+    if (rc != SLC_ERR_UNSUPPORTED) return rc;
+  }
   switch (dtype) {
     case SLC_F32:
       return launch_generic<float>(input, weight, bias, output, M, N, K,

@@ -286,6 +286,30 @@ def test_linear_fp32(gpu, rows):
     assert_fp32_close(y, ref.linear(x, w, b))
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17, 33, 64, 65, 129, 300])
+@pytest.mark.parametrize("n,k,bias", [(896, 896, True), (1027, 32, False), (130, 4864, True), (33, 100, True),
+                                      (65, 30, False)])
+def test_linear_fp32_matrix_cores(gpu, rows, n, k, bias):
+    """fp32 linears on the matrix cores (and the shapes they leave to the
+    generic kernel) stay within the error of any fp32 accumulation order."""
+
+    from stateful_llm_compiler_hip.backends import hip_linear
+
+    announce(f"linear fp32 M={rows} N={n} K={k} bias={bias}")
+    g = generator(rows + n + k)
+    x, w = torch.randn(rows, k, generator=g), torch.randn(n, k, generator=g)
+    b = torch.randn(n, generator=g) if bias else None
+    actual = hip_linear(x.to(gpu), w.to(gpu), None if b is None else b.to(gpu)).cpu().double()
+    exact, terms = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    if b is not None:
+        exact, terms = exact + b.double(), terms + b.double().abs()
+    # Every product and every partial sum is rounded at most once to fp32:
+    # (K + 1) * 2^-24 * sum|terms| bounds any order (Higham, 2002, section 3.1).
+    assert ((actual - exact).abs() <= (k + 1) * 2.0**-24 * terms).all()
+    # Rounding errors add like a random walk: twice sqrt(K) of them in the norm.
+    assert (actual - exact).norm() <= 2 * k**0.5 * 2.0**-24 * terms.norm()
+
+
 # -------------------------------------------------------- prefill attention
 
 
