@@ -174,6 +174,14 @@ int gemm_residual(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t 
 // (nothing launched) for shapes its kernels do not take.
 int linear_f32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
                int64_t x_rs, int64_t y_rs, hipStream_t stream);
+// fp32 prefill attention on the fp32 matrix cores (prefill_f32.hip), strides
+// in the order of slc_hip_prefill_attention; SLC_ERR_UNSUPPORTED (nothing
+// launched) for shapes it does not take.
+int prefill_attention_f32(const float* query, const float* key, const float* value, const void* mask,
+                          int mask_dtype, const unsigned char* tile_class, float* output,
+                          int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t tokens,
+                          int64_t head_dim, int causal, const int64_t* strides, float scale,
+                          hipStream_t stream);
 bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                           int dtype);
 int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,

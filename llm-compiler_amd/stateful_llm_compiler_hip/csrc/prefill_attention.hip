@@ -20,7 +20,7 @@
 //    single ds_read_b128 / register reads.
 //  * Causal: tiles entirely in a wave's future are skipped (and workgroups
 //    are launched heaviest-first); the diagonal tile is masked per element.
-// fp32 and other shapes take a simple wave-per-query kernel.
+// fp32 runs in prefill_f32.hip; other shapes take a simple wave-per-query kernel.
 #include "prefill_v2.hpp"
 
 namespace {
@@ -535,6 +535,13 @@ extern "C" int slc_hip_prefill_attention_classes(
     }
     return causal ? dispatch_mask<slc::f16_t, true>(query, key, value, mask, mask_dtype, output, batch, T_, static_cast<int>(q_heads), groups, st, scale, s)
                   : dispatch_mask<slc::f16_t, false>(query, key, value, mask, mask_dtype, output, batch, T_, static_cast<int>(q_heads), groups, st, scale, s);
+  }
+  if (dtype == SLC_F32) {
+    const int rc = slc_host::prefill_attention_f32(
+        static_cast<const float*>(query), static_cast<const float*>(key),
+        static_cast<const float*>(value), mask, mask_dtype, mask_tile_classes,
+        static_cast<float*>(output), batch, q_heads, kv_heads, tokens, head_dim, causal, st, scale, s);
+    if (rc != SLC_ERR_UNSUPPORTED) return rc;
   }
   switch (dtype) {
     case SLC_F32:

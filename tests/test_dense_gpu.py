@@ -499,6 +499,43 @@ def test_prefill_fp32_generic(gpu):
     assert_fp32_close(actual, expected)
 
 
+@pytest.mark.parametrize("tokens", [1, 16, 63, 64, 65, 200])
+@pytest.mark.parametrize("kind,causal,mask_dtype", [
+    ("none", True, torch.float32), ("none", False, torch.float32), ("causal", False, torch.float32),
+    ("random", True, torch.float32), ("random", False, torch.bfloat16), ("zeros", False, torch.float16)])
+@pytest.mark.parametrize("order", ["online", "exact"])
+def test_prefill_fp32_matrix_cores(gpu, tokens, kind, causal, mask_dtype, order):
+    announce(f"prefill fp32 T={tokens} mask={kind} {mask_dtype} causal={causal} order={order}")
+    q_heads, kv_heads = (14, 2) if tokens != 63 else (3, 1)
+    actual, expected = _prefill_case(gpu, 2, tokens, torch.float32, tokens, mask_kind=kind, causal=causal,
+                                     q_heads=q_heads, kv_heads=kv_heads, mask_dtype=mask_dtype,
+                                     softmax_order=order)
+    assert_fp32_close(actual, expected)
+
+
+def test_prefill_fp32_masked_tiles_and_rows(gpu):
+    # Padding that rules out whole key tiles, and a batch row with nothing to
+    # attend to: NaN there, as the reference's softmax over an all -inf row.
+    from stateful_llm_compiler_hip.backends import hip_prefill_attention
+
+    announce("prefill fp32 dead tiles and an empty row T=300")
+    g = generator(12)
+    tokens = 300
+    q, k, v = (torch.randn(3, h, tokens, 64, generator=g) for h in (14, 2, 2))
+    at = torch.arange(tokens)
+    hidden = (at.view(1, 1, -1) > at.view(1, -1, 1)) | (at.view(1, 1, -1) < torch.tensor([0, 130, 0]).view(3, 1, 1))
+    hidden = hidden & (at.view(1, 1, -1) != at.view(1, -1, 1))
+    hidden[2, 70] = True
+    mask = torch.zeros(3, 1, tokens, tokens).masked_fill(hidden.unsqueeze(1), float("-inf"))
+    expected = ref.prefill_attention(q, k, v, mask, groups=7, scale=0.125, causal=False)
+    actual = hip_prefill_attention(q.to(gpu), k.to(gpu), v.to(gpu), mask.to(gpu), scale=0.125,
+                                   softmax_order="exact").cpu()
+    empty = torch.isnan(expected)
+    assert bool(empty[2, :, 70].all()) and int(empty.sum()) == 14 * 64
+    assert torch.equal(torch.isnan(actual), empty)
+    assert_fp32_close(actual[~empty], expected[~empty])
+
+
 def test_prefill_fp16_head_dim_128_generic(gpu):
     announce("prefill fp16 D=128 (generic)")
     actual, expected = _prefill_case(gpu, 1, 40, torch.float16, 9, mask_kind="none", causal=True, q_heads=4, head_dim=128)
