@@ -182,6 +182,19 @@ int prefill_attention_f32(const float* query, const float* key, const float* val
                           int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t tokens,
                           int64_t head_dim, int causal, const int64_t* strides, float scale,
                           hipStream_t stream);
+// fp32 decode attention on the fp32 matrix cores (decode_f32.hip), strides in
+// the order of slc_hip_decode_attention.  A workspace or counter array smaller
+// than decode_f32_chunks asks for costs the split, not the call.
+// SLC_ERR_UNSUPPORTED (nothing launched) for shapes it does not take.
+bool decode_f32_eligible(int64_t head_dim, int64_t groups);
+int64_t decode_f32_chunks(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
+                          int64_t mask_len);
+int decode_attention_f32(const float* query, const float* kb, const float* vb, const void* lengths,
+                         int lengths_dtype, const void* mask, int mask_dtype, float* output,
+                         void* workspace, int64_t workspace_bytes, int* counters,
+                         int64_t num_counters, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                         int64_t head_dim, int64_t capacity, int64_t mask_len,
+                         const int64_t* strides, float scale, hipStream_t stream);
 bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                           int dtype);
 int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,

@@ -25,7 +25,8 @@
 //    workgroup -- an L2 write-back -- which measured several times slower than
 //    the extra launch.)
 //  * Loops stop at the batch's own length, not at the capacity.
-// Other dtypes/shapes take a straightforward wave-per-token kernel.
+// fp32 runs in decode_f32.hip; other shapes take a straightforward
+// wave-per-token kernel.
 #include <algorithm>
 #include <climits>
 #include <mutex>
@@ -220,6 +221,11 @@ extern "C" int64_t slc_hip_decode_attention_workspace_size(
       q_heads % kv_heads != 0) {
     return 0;
   }
+  if (dtype == SLC_F32)
+    return slc_host::decode_f32_eligible(head_dim, q_heads / kv_heads)
+               ? partial_bytes(batch, q_heads, head_dim,
+                               slc_host::decode_f32_chunks(batch, q_heads, kv_heads, head_dim, mask_len))
+               : 0;
   // The online split needs at least what the exact single-chunk form does.
   // Enough for either split (the balanced one may decline at the call's
   // capacity and take the fixed-chunk grid).
@@ -333,6 +339,14 @@ extern "C" int slc_hip_decode_attention(
   }
   SLC_REQUIRE(batch * q_heads <= 0x7fffffff,
               "slc_hip_decode_attention: grid too large");
+  if (dtype == SLC_F32) {
+    const int rc = slc_host::decode_attention_f32(
+        static_cast<const float*>(query), static_cast<const float*>(key_buffer),
+        static_cast<const float*>(value_buffer), lengths, lengths_dtype, mask, mask_dtype,
+        static_cast<float*>(output), workspace, workspace_bytes, counters, num_counters, batch,
+        q_heads, kv_heads, head_dim, capacity, ml, st, scale, s);
+    if (rc != SLC_ERR_UNSUPPORTED) return rc;
+  }
   switch (dtype) {
     case SLC_F32:
       return launch_generic<float>(query, key_buffer, value_buffer, lengths,

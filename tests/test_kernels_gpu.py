@@ -384,6 +384,29 @@ def test_decode_attention_positions_past_length_are_ignored(gpu):
 # ------------------------------------------------------------------ rms_norm
 
 
+@pytest.mark.parametrize("batch,q_heads,kv_heads,head_dim,capacity,lengths,mask_kind,mask_dtype", [
+    (1, 14, 2, 64, 1, [1], "zeros", torch.float32),
+    (3, 14, 2, 64, 65, [7, 31, 65], "random", torch.float32),       # one chunk
+    (4, 14, 2, 64, 129, [0, 128, 129, 16], "random", torch.bfloat16),  # two chunks; an empty row (NaN)
+    (2, 4, 2, 128, 1000, [1000, 17], "random", torch.float16),
+    (5, 16, 1, 64, 3001, [1, 15, 64, 2999, 3001], "random", torch.float32),  # 16 heads, many chunks
+    (300, 3, 3, 64, 140, None, "zeros", torch.float32),             # more pairs than workgroups: one chunk
+])
+@pytest.mark.parametrize("order", ["online", "exact"])
+@pytest.mark.parametrize("layout", ["bshd", "bhsd"])
+def test_decode_fp32_matrix_cores(gpu, batch, q_heads, kv_heads, head_dim, capacity, lengths, mask_kind, mask_dtype,
+                                  order, layout):
+    announce(f"decode fp32 B={batch} QH={q_heads} KVH={kv_heads} D={head_dim} cap={capacity} {order} {layout}")
+    if lengths is None:
+        lengths = torch.randint(1, capacity + 1, (batch,), generator=generator(3)).tolist()
+    actual, expected = _decode_case(gpu, batch, q_heads, kv_heads, head_dim, capacity, lengths, torch.float32,
+                                    capacity, mask_kind=mask_kind, mask_dtype=mask_dtype, softmax_order=order,
+                                    layout=layout)
+    empty = torch.isnan(expected)
+    assert torch.equal(torch.isnan(actual), empty)
+    assert_fp32_close(actual[~empty], expected[~empty])
+
+
 @pytest.mark.parametrize("waves", [None, 1, 4])
 @pytest.mark.parametrize("rows", [1, 8, 64, 512, 32768])
 def test_rms_norm_bf16_round_before_weight(gpu, rows, waves):
