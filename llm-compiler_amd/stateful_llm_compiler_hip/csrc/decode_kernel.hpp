@@ -985,28 +985,35 @@ bool mfma_eligible(int dtype, int64_t head_dim, int64_t groups) {
          (head_dim == 64 || head_dim == 128) && groups <= kMaxGroups;
 }
 
-#ifndef SLC_DECODE_MIN_CHUNK
-#define SLC_DECODE_MIN_CHUNK 256
-#endif
-
-// Sequence chunk of the split-sequence grid: the smallest power-of-two
-// multiple of the workgroup's 128-token sweep that keeps the grid at about one
-// workgroup per CU (256 CUs on MI355X); longer chunks amortise the per-wave
-// pipeline fill and keep the partials small.
+// Sequence chunk of the split-sequence grid, a multiple of the workgroup's
+// 128-token sweep.  A workgroup takes about 7 ns per token of its chunk, a
+// split about 4 us for publishing and merging and 0.2 us per chunk more, and
+// past one workgroup per CU (256 on MI355X) every further release write-back
+// costs more than it saves.  So (graphs of back-to-back calls, microseconds):
+//  * one chunk where splitting gains less than the merge: masks up to 640
+//    tokens (B1 L512 8.0 -> 6.0, B48 L600 11.4 -> 8.2), and up to 1024 where
+//    the grid leaves two chunks at most (B64 L1024 12.9 -> 11.8);
+//  * else equal chunks of at least 256 tokens, at most one workgroup per CU
+//    (B20 L17963 D128: six chunks of 3072 tokens 68, five of 4096 80);
+//  * and chunk^2 >= 16 mask_len, which balances the chunk against the merge
+//    for few long sequences (B1 L32768: 128 chunks of 256 34.8, 32 of 1024
+//    19.3; B1 L16384 22.3 -> 16.4).
 int64_t choose_chunk(int64_t batch, int64_t kv_heads, int64_t mask_len,
                      int64_t split_tokens) {
   const int64_t sweep = kWaves * kTile;
+  auto sweeps = [&](int64_t tokens) { return slc_host::ceil_div(tokens, sweep) * sweep; };
   int64_t chunk;
   if (split_tokens > 0) {
-    chunk = slc_host::ceil_div(split_tokens, sweep) * sweep;
+    chunk = sweeps(split_tokens);
   } else {
-    const int64_t target_groups = 256;
-    chunk = SLC_DECODE_MIN_CHUNK;
-    // Stop at one chunk per sequence: with more (batch, kv-head) pairs than
-    // the target the grid is already that wide.
-    while (chunk < mask_len &&
-           batch * kv_heads * slc_host::ceil_div(mask_len, chunk) > target_groups) {
-      chunk *= 2;
+    const int64_t most = std::max<int64_t>(1, 256 / std::max<int64_t>(1, batch * kv_heads));
+    if (mask_len <= 640 || (most <= 2 && mask_len <= 1024)) {
+      chunk = sweeps(mask_len);
+    } else {
+      chunk = std::max<int64_t>(256, sweeps(slc_host::ceil_div(mask_len, most)));
+      while (chunk * chunk < 16 * mask_len) chunk += sweep;
+      // Equal chunks: as many as that leaves, no longer than they need be.
+      chunk = sweeps(slc_host::ceil_div(mask_len, slc_host::ceil_div(mask_len, chunk)));
     }
   }
   // The merge keeps every chunk's weight of a (batch, kv-head) in LDS.

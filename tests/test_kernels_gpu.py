@@ -197,6 +197,18 @@ def test_decode_attention_layouts_and_length_dtypes(gpu, layout, length_dtype, s
     assert_bf16_close(actual, expected)
 
 
+@pytest.mark.parametrize("batch,max_len", [(1, 640), (1, 641), (64, 1024), (64, 1025), (3, 9001), (1, 20000)])
+def test_decode_bf16_automatic_chunks(gpu, batch, max_len):
+    # Either side of the one-chunk limits, and chunk lengths that are no power
+    # of two and do not divide the mask.
+    announce(f"decode bf16 automatic chunks B={batch} L={max_len}")
+    lengths = torch.randint(1, max_len + 1, (batch,), generator=generator(max_len)).tolist()
+    lengths[0] = max_len
+    actual, expected = _decode_case(gpu, batch, 14, 2, 64, max_len, lengths, torch.bfloat16, 90 + batch,
+                                    mask_kind="random")
+    assert_bf16_close(actual, expected)
+
+
 @pytest.mark.parametrize("split", [128, 256, 2048])
 def test_decode_attention_forced_split(gpu, split):
     announce(f"decode bf16 split_tokens={split}")
