@@ -147,12 +147,12 @@ def hip_norm_linear_swiglu(
 
 def _linear_group(x: torch.Tensor, weights: Sequence[torch.Tensor],
                   biases: Sequence[torch.Tensor | None]) -> list[torch.Tensor] | None:
-    """Prefill-sized ``[linear(x, w, b) ...]`` in one launch, or None (nothing
+    """``[linear(x, w, b) ...]`` past the norm kernels' rows in one launch, or None (nothing
     launched) when that kernel does not take the shapes."""
 
     hidden = x.shape[-1]
     rows = x.numel() // hidden if hidden else 0
-    if (not x.is_cuda or not x.is_contiguous() or rows <= 64
+    if (not x.is_cuda or not x.is_contiguous() or rows <= MAX_FUSED_ROWS
             or x.dtype not in (torch.bfloat16, torch.float16)
             or any(b is not None and (b.dtype != x.dtype or not b.is_contiguous()) for b in biases)):
         return None
@@ -178,12 +178,12 @@ def _linear_group(x: torch.Tensor, weights: Sequence[torch.Tensor],
 
 def _linear_swiglu(x: torch.Tensor, gate_weight: torch.Tensor,
                    up_weight: torch.Tensor) -> torch.Tensor | None:
-    """Prefill-sized ``swiglu(linear(x, gate), linear(x, up))`` in one kernel,
+    """``swiglu(linear(x, gate), linear(x, up))`` past the norm kernels' rows in one kernel,
     or None (nothing launched) when that kernel does not take the shape."""
 
     hidden = x.shape[-1]
     rows = x.numel() // hidden if hidden else 0
-    if (not x.is_cuda or not x.is_contiguous() or rows <= 64
+    if (not x.is_cuda or not x.is_contiguous() or rows <= MAX_FUSED_ROWS
             or x.dtype not in (torch.bfloat16, torch.float16)):
         return None
     features = gate_weight.shape[0]

@@ -16,7 +16,7 @@
 //  * rope_kv_store       rope -> kv_store of the rotated keys and the values;
 //                        the rotated queries are written out.
 //
-// slc_hip_linear runs its decode-sized (<= 32 rows) cases on this same kernel
+// slc_hip_linear runs its decode-sized (<= 64 rows) cases on this same kernel
 // (rows_linear), so a fused op and the ops it replaces share the K split over
 // the waves, the MFMA order and the partial-sum order, hence the same bits.
 // Semantics: src/stateful_llm_compiler/execution.py:674-692 (rms_norm),
@@ -65,10 +65,16 @@ enum Epilogue { kStore = 0, kResidual = 1, kSwiglu = 2 };
 
 // Waves per workgroup (the K split): 16 from K = 512 (more loads in flight
 // per CU: Qwen2 decode SwiGLU 8.1 against 8.9 us with 8, down projection 7.3
-// against 8.0), else 8.  It depends on K alone, so the fused ops and the
-// single linears they replace split K the same way.
-__host__ __device__ constexpr int waves_for(int k) { return k >= 512 ? 16 : 8; }
-constexpr int kMaxRows = 32;     // rows (batch x tokens) the fused kernels take
+// against 8.0), else 8.  Past 32 rows a wave's accumulators and input operands
+// need the registers of an 8-wave workgroup (16 waves measured the same where
+// they fit: M48 N896 K4864 17.2 us both ways).  It depends on K and the rows
+// alone, so the fused ops and the single linears they replace split K the same
+// way.
+__host__ __device__ constexpr int waves_for(int k, int rows) {
+  return k >= 512 && rows <= 32 ? 16 : 8;
+}
+constexpr int kMaxRows = 32;     // rows (batch x tokens) the kernels with a norm take
+constexpr int kMaxPlainRows = 64;  // rows the kernels without one take
 constexpr int kMaxMatrices = 3;
 
 struct FusedArgs {
@@ -360,7 +366,7 @@ template <typename T, int NV, int EPI>
 int launch_rows(FusedArgs& a, hipStream_t stream) {
   const int blocks = a.block_end[kMaxMatrices - 1];
   const int nw = EPI == kSwiglu ? 2 : 1;
-  const int kw = waves_for(a.hidden);
+  const int kw = waves_for(a.hidden, a.rows);
   const int tiles = a.feat > 16 ? 2 : 1;
   auto go = [&](auto kernel, int mb) {
     const int xs_bytes = NV > 0 ? mb * 16 * norm_row(a.hidden) * 2 : 0;
@@ -384,6 +390,22 @@ int launch_rows(FusedArgs& a, hipStream_t stream) {
   constexpr int U1 = EPI == kSwiglu ? 4 : 8, U2 = EPI == kSwiglu ? 2 : 4;
   // 16 waves: half the k-steps per wave, half the prefetch depth.
   constexpr int V1 = U1 / 2, V2 = U2 / 2;
+  if constexpr (NV == 0) {
+    // 33 .. 64 rows: three or four blocks of 16 input rows share every weight
+    // read; the input rows come from the cache, each wave its own k-slice
+    // (which bounds long K: each further block of 16 rows costs 4 us at K =
+    // 4864, whether 56 or 224 workgroups share the features).  M48 N4864 K896
+    // 10.0 -> 7.4 us, M48 N896 K4864 19 -> 17, and the MLP's five launches
+    // become three: 54 -> 29 us at 48 rows.
+    if (a.rows > 32) {
+      constexpr int W = EPI == kSwiglu ? 1 : 2;  // k-steps in flight, within the registers
+      if (tiles == 2)
+        return a.rows <= 48 ? go(fused_rows_kernel<T, 3, 8, W, 0, EPI, 2>, 3)
+                            : go(fused_rows_kernel<T, 4, 8, W, 0, EPI, 2>, 4);
+      return a.rows <= 48 ? go(fused_rows_kernel<T, 3, 8, 2 * W, 0, EPI, 1>, 3)
+                          : go(fused_rows_kernel<T, 4, 8, 2 * W, 0, EPI, 1>, 4);
+    }
+  }
   if (kw == 16) {
     if (tiles == 2) {
       if (a.rows <= 16) return go(fused_rows_kernel<T, 1, 16, V1 / 2, NV, EPI, 2>, 1);
@@ -740,9 +762,77 @@ int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
 
 bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                           int dtype) {
-  return (dtype == SLC_BF16 || dtype == SLC_F16) && rows >= 1 && rows <= kMaxRows &&
+  return (dtype == SLC_BF16 || dtype == SLC_F16) && rows >= 1 && rows <= kMaxPlainRows &&
          K % 8 == 0 && K >= 8 && x_rs % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-         N <= (1 << 24);
+         N <= (1 << 24) && (rows <= kMaxRows || (N + 15) / 16 < kWideBlocks);
+}
+
+// The fused forms for 33 .. 64 rows (their norm, if any, ran before): up to
+// three linears of one input, the SwiGLU pair, the linear with its residual
+// add.  SLC_ERR_UNSUPPORTED (nothing launched) for shapes they do not take.
+int rows_group(const void* x, int64_t x_rs, int64_t rows, int64_t K, int count,
+               const void* const* w, const void* const* bias, void* const* y, const int64_t* n,
+               const int64_t* y_rs, int dtype, hipStream_t stream) {
+  FusedArgs a{};
+  a.x = x;
+  a.x_rs = x_rs;
+  a.rows = static_cast<int>(rows);
+  a.hidden = static_cast<int>(K);
+  for (int i = 0; i < count; ++i) {
+    if (w[i] == nullptr || y[i] == nullptr || n[i] < 1 || y_rs[i] < n[i] ||
+        (reinterpret_cast<uintptr_t>(w[i]) & 15) != 0 ||
+        !rows_linear_eligible(x, x_rs, rows, K, n[i], dtype))
+      return SLC_ERR_UNSUPPORTED;
+    a.w[i] = w[i];
+    a.bias[i] = bias[i];
+    a.y[i] = y[i];
+    a.n[i] = static_cast<int>(n[i]);
+    a.y_rs[i] = y_rs[i];
+  }
+  assign_blocks(a, count);
+  return dispatch_rows<kStore>(a, dtype, stream);
+}
+
+int rows_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
+                const void* w_gate, const void* w_up, void* y, int64_t y_rs, int dtype,
+                hipStream_t stream) {
+  const uint64_t bits = reinterpret_cast<uintptr_t>(w_gate) | reinterpret_cast<uintptr_t>(w_up);
+  if ((bits & 15) != 0 || y_rs < N || !rows_linear_eligible(x, x_rs, rows, K, N, dtype))
+    return SLC_ERR_UNSUPPORTED;
+  FusedArgs a{};
+  a.x = x;
+  a.x_rs = x_rs;
+  a.rows = static_cast<int>(rows);
+  a.hidden = static_cast<int>(K);
+  a.w[0] = w_gate;
+  a.w[1] = w_up;
+  a.y[0] = y;
+  a.n[0] = static_cast<int>(N);
+  a.y_rs[0] = y_rs;
+  assign_blocks(a, 1);
+  return dispatch_rows<kSwiglu>(a, dtype, stream);
+}
+
+int rows_residual(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N, const void* w,
+                  const void* bias, const void* residual, int64_t r_rs, void* y, int64_t y_rs,
+                  int dtype, hipStream_t stream) {
+  if ((reinterpret_cast<uintptr_t>(w) & 15) != 0 || y_rs < N || r_rs < N ||
+      !rows_linear_eligible(x, x_rs, rows, K, N, dtype))
+    return SLC_ERR_UNSUPPORTED;
+  FusedArgs a{};
+  a.x = x;
+  a.x_rs = x_rs;
+  a.rows = static_cast<int>(rows);
+  a.hidden = static_cast<int>(K);
+  a.w[0] = w;
+  a.bias[0] = bias;
+  a.y[0] = y;
+  a.n[0] = static_cast<int>(N);
+  a.y_rs[0] = y_rs;
+  a.residual = residual;
+  a.r_rs = r_rs;
+  assign_blocks(a, 1);
+  return dispatch_rows<kResidual>(a, dtype, stream);
 }
 
 }  // namespace slc_host
@@ -827,6 +917,10 @@ extern "C" int slc_hip_linear_residual(const void* x, int64_t x_rs, int64_t rows
     // Prefill-sized: the tile kernel with the residual in its store epilogue.
     SLC_REQUIRE(x && weight && residual && y && in_features >= 1 && out_features >= 1,
                 "%s: bad operands", what);
+    if (rows <= kMaxPlainRows)
+      return slc_host::rows_residual(x, x_rs, rows, in_features, out_features, weight, bias,
+                                     residual, residual_rs, y, y_rs, dtype,
+                                     static_cast<hipStream_t>(stream));
     return slc_host::gemm_residual(x, x_rs, rows, in_features, out_features, weight, bias,
                                    residual, residual_rs, y, y_rs, dtype,
                                    static_cast<hipStream_t>(stream));

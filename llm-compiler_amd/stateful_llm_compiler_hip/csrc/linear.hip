@@ -1137,9 +1137,10 @@ int launch_ring_tile(int tile, const void* x, const void* w, const void* bias, v
 template <typename T>
 int dispatch_mfma(const void* x, const void* w, const void* bias, void* y, int M,
                   int N, int K, int64_t x_rs, int64_t y_rs, hipStream_t s, int tile = SLC_TILE_AUTO) {
-  // Up to 32 rows: the decode-step linear kernel the fused ops share.
+  // Up to 64 rows: the decode-step linear kernel the fused ops share (a
+  // vocabulary-wide output past 32 rows: the skinny kernel below).
   const int dtype = sizeof(T) == 2 && std::is_same<T, slc::bf16_t>::value ? SLC_BF16 : SLC_F16;
-  if (M <= 32 && slc_host::rows_linear_eligible(x, x_rs, M, K, N, dtype))
+  if (M <= 64 && slc_host::rows_linear_eligible(x, x_rs, M, K, N, dtype))
     return slc_host::rows_linear(x, x_rs, M, K, N, w, bias, y, y_rs, dtype, s);
   if (M <= 16) return launch_skinny<T, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
   if (M <= 32) return launch_skinny<T, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
@@ -1224,6 +1225,8 @@ int gemm_residual(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t 
 int gemm_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                 const void* w_gate, const void* w_up, void* y, int64_t y_rs, int dtype,
                 hipStream_t stream) {
+  if (rows > 32 && rows <= 64)
+    return rows_swiglu(x, x_rs, rows, K, N, w_gate, w_up, y, y_rs, dtype, stream);
   const uint64_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w_gate) |
                         reinterpret_cast<uintptr_t>(w_up) | reinterpret_cast<uintptr_t>(y);
   const bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 64 && (bits & 15) == 0 &&
@@ -1266,6 +1269,8 @@ int gemm_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
 int gemm_group(const void* x, int64_t x_rs, int64_t rows, int64_t K, int count,
                const void* const* w, const void* const* bias, void* const* y,
                const int64_t* n, const int64_t* y_rs, int dtype, hipStream_t stream) {
+  if (rows > 32 && rows <= 64)
+    return rows_group(x, x_rs, rows, K, count, w, bias, y, n, y_rs, dtype, stream);
   bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 64 && count >= 1 && count <= 3 &&
             K % kBK == 0 && x_rs % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
             128 * x_rs * 2 < (int64_t{1} << 31) && rows < (int64_t{1} << 31);

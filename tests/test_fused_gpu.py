@@ -106,6 +106,36 @@ def test_linear_residual_matches_linear_then_add(gpu, rows, n, k):
     assert_bitwise_equal(got, want)
 
 
+@pytest.mark.parametrize("rows", [33, 48, 49, 64, 65])
+@pytest.mark.parametrize("hidden,features,dtype", [(896, 4864, torch.bfloat16), (4864, 896, torch.float16),
+                                                   (2048, 5000, torch.bfloat16), (72, 40, torch.bfloat16)])
+def test_plain_fused_ops_past_the_norm_rows(gpu, rows, hidden, features, dtype):
+    """33 to 64 rows: the fused ops run without their norm on the decode
+    kernel, bit for bit the single linears (which match float64)."""
+    announce(f"fused ops rows={rows} hidden={hidden} features={features} {dtype}")
+    g = generator(rows + features)
+    x = _t(g, rows, 1, hidden, dtype=dtype, device=gpu)
+    ws = [_t(g, n, hidden, dtype=dtype, scale=0.02, device=gpu) for n in (features, features, 24)]
+    bs = [_t(g, features, dtype=dtype, scale=0.1, device=gpu), None, None]
+    single = [hip_linear(x, w, b) for w, b in zip(ws, bs)]
+    for got, want in zip(hip_norm_linear_group(x, None, ws, bs, epsilon=1e-6), single):
+        assert_bitwise_equal(got, want)
+    r = _t(g, rows, 1, features, dtype=dtype, device=gpu)
+    assert_bitwise_equal(hip_linear_residual(x, ws[0], bs[0], r), hip_add(r, single[0]))
+    if hidden <= 2048:
+        nw = _t(g, hidden, dtype=dtype, scale=0.5, device=gpu) + 1
+        xn = hip_rms_norm(x, nw, epsilon=1e-6, round_before_weight=True)
+        assert_bitwise_equal(hip_norm_linear_swiglu(x, nw, ws[0], ws[1], epsilon=1e-6),
+                             hip_swiglu(hip_linear(xn, ws[0]), hip_linear(xn, ws[1])))
+    exact = x.double().cpu() @ ws[1].double().cpu().T
+    terms = x.double().abs().cpu() @ ws[1].double().abs().cpu().T
+    # One rounding to the type (half a unit: 2^-8 or 2^-11 of the value), any
+    # order of an fp32 sum, and fp16's subnormal spacing.
+    unit = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    bound = unit * exact.abs() + (hidden + 1) * 2.0**-24 * terms + 2.0**-24
+    assert ((single[1].double().cpu() - exact).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("tokens", [1, 5])
 def test_rope_kv_store_matches_rope_then_store(gpu, tokens):
     announce(f"rope_kv_store tokens={tokens}")
