@@ -593,10 +593,8 @@ int launch_wide(FusedArgs& a, hipStream_t stream) {
   if (a.rows <= 16 && SLC_WIDE_XL && a.hidden % 8 == 0 && x_aligned && x_bytes <= 32 * 1024) {
     hipLaunchKernelGGL((wide_rows_kernel<T, 1, SLC_WIDE_U, true>), dim3(blocks), dim3(256),
                        static_cast<unsigned>(x_bytes), stream, a);
-  } else if (a.rows <= 16) {
-    hipLaunchKernelGGL((wide_rows_kernel<T, 1, SLC_WIDE_U>), dim3(blocks), dim3(256), 0, stream, a);
   } else {
-    hipLaunchKernelGGL((wide_rows_kernel<T, 2, 4>), dim3(blocks), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((wide_rows_kernel<T, 1, SLC_WIDE_U>), dim3(blocks), dim3(256), 0, stream, a);
   }
   return slc_host::check_launch("decode linear (wide)");
 }
@@ -764,7 +762,7 @@ bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, 
                           int dtype) {
   return (dtype == SLC_BF16 || dtype == SLC_F16) && rows >= 1 && rows <= kMaxPlainRows &&
          K % 8 == 0 && K >= 8 && x_rs % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-         N <= (1 << 24) && (rows <= kMaxRows || (N + 15) / 16 < kWideBlocks);
+         N <= (1 << 24) && (rows <= 16 || (N + 15) / 16 < kWideBlocks);
 }
 
 // The fused forms for 33 .. 64 rows (their norm, if any, ran before): up to

@@ -1092,19 +1092,31 @@ inline bool stream_grid(int64_t tiles) {
          tiles >= int64_t{SLC_STREAM_MIN_ROUNDS} * slc_host::device_cu_count();
 }
 
-// Ring-kernel tile for a shape when the caller leaves it to the library, by
-// the number of 128 x 128 tiles the shape has: 256 x 128 from 300 of them
-// (the larger tile reads less per flop once the grid is a few rounds deep),
-// 128 x 128 from 128 (half a round on 256 CUs), then 128 x 64 while that
-// grid has 192 workgroups, else 64 x 64 (small grids: the deep ring hides the
-// latency of K's many k-tiles).  The winners measured on MI355X at the
-// Qwen2-0.5B projection shapes for M = 128 .. 32768.
+// Ring-kernel tile for a shape when the caller leaves it to the library: the
+// smallest tile whose grid is at most one round of the CUs (a small grid is
+// bound by the latency of K's many k-tiles, which does not grow with the
+// grid until a second round starts: M1000 N896 K4864 64 x 64 19.5 us, M1365
+// 34.6, there 128 x 64 26.1), then 128 x 128, and 256 x 128 from 300 tiles of
+// 128 x 128 (it reads less per flop once the grid is a few rounds deep).  The
+// winners measured on MI355X at the Qwen2-0.5B projection shapes for M = 65 ..
+// 32768.
 inline int auto_ring_tile(int64_t M, int64_t n_tiles128) {
+  const int64_t cus = slc_host::device_cu_count();
   const int64_t n128 = ((M + 127) / 128) * n_tiles128;
-  if (n128 >= 300) return SLC_TILE_R256X128;
-  if (n128 >= 128) return SLC_TILE_R128X128;
-  if (2 * n128 >= 192) return SLC_TILE_R128X64;
-  return SLC_TILE_R64X64;
+  if (((M + 63) / 64) * 2 * n_tiles128 <= cus) return SLC_TILE_R64X64;
+  if (2 * n128 <= cus) return SLC_TILE_R128X64;
+  return n128 >= 300 ? SLC_TILE_R256X128 : SLC_TILE_R128X128;
+}
+
+// Vocabulary-wide outputs write as many bytes as they read, and three
+// register-staged 128 x 128 workgroups per CU overlap one's stores with the
+// others' loads: with up to 128 rows they stream the weights (M65 N151936
+// 51.9 us, the 256 x 128 ring 82.2, the skinny kernel 180 at M64), and they
+// win whenever 256-row tiles would leave half a tile empty (M300 128.5 against
+// 150.4; M1000 334.5 against 328.7).
+constexpr int kWideOutputs = 16384;
+inline bool wide_on_register_tiles(int64_t M, int64_t N) {
+  return N >= kWideOutputs && ((M + 127) / 128) % 2 == 1;
 }
 
 // One of the ring tiles; kNoResidualPath (nothing launched) where the shape
@@ -1138,17 +1150,21 @@ template <typename T>
 int dispatch_mfma(const void* x, const void* w, const void* bias, void* y, int M,
                   int N, int K, int64_t x_rs, int64_t y_rs, hipStream_t s, int tile = SLC_TILE_AUTO) {
   // Up to 64 rows: the decode-step linear kernel the fused ops share (a
-  // vocabulary-wide output past 32 rows: the skinny kernel below).
+  // vocabulary-wide output past 16 rows: the tiles below).
   const int dtype = sizeof(T) == 2 && std::is_same<T, slc::bf16_t>::value ? SLC_BF16 : SLC_F16;
   if (M <= 64 && slc_host::rows_linear_eligible(x, x_rs, M, K, N, dtype))
     return slc_host::rows_linear(x, x_rs, M, K, N, w, bias, y, y_rs, dtype, s);
   if (M <= 16) return launch_skinny<T, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-  if (M <= 32) return launch_skinny<T, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-  if (M <= 64) return launch_skinny<T, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
+  if (M <= 32 && N < kWideOutputs) return launch_skinny<T, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
+  if (M <= 64) {
+    if (N >= kWideOutputs) return launch_mfma<T, 128, 128, 2, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
+    return launch_skinny<T, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
+  }
   // Tile variants (a profile plan picks one): every tile accumulates each
   // output's k range in the same order, 32 k at a time on one MFMA chain, so
   // the variants differ in speed only, never in a bit of the result.
-  if (tile == SLC_TILE_AUTO) tile = auto_ring_tile(M, (N + 127) / 128);
+  if (tile == SLC_TILE_AUTO)
+    tile = wide_on_register_tiles(M, N) ? SLC_TILE_128X128 : auto_ring_tile(M, (N + 127) / 128);
   switch (tile) {
     case SLC_TILE_128X64:
       return launch_mfma<T, 128, 64, 2, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
