@@ -377,7 +377,7 @@ __device__ __forceinline__ void xcd_tile(int n_tiles, int m_tiles, int& m_blk, i
 }
 
 template <typename T, int BM, int BN, int CWM, int CWN, int PW, int S, int GM = 8,
-          bool DUAL = false, bool GROUP = false>
+          bool DUAL = false, bool GROUP = false, int KT = 1>
 __global__ __launch_bounds__((CWM * CWN + PW) * 64) void linear_ring_kernel(
     const T* __restrict__ x, const T* __restrict__ w_arg, const T* __restrict__ bias_arg,
     T* __restrict__ y_arg, int M, int N_arg, int K, int64_t x_rs, int64_t y_rs_arg,
@@ -391,8 +391,11 @@ __global__ __launch_bounds__((CWM * CWN + PW) * 64) void linear_ring_kernel(
   constexpr int FM = TM / 16;
   constexpr int FN = TN / 16;
   constexpr int XB = BM * kBK * 2;   // bytes of an X tile
-  constexpr int kStage = (BM + BN) * kBK * 2;
-  constexpr int kOps = (BM + BN) / 8 / PW;  // 1 KB DMA instructions per producer wave per tile
+  constexpr int kSub = (BM + BN) * kBK * 2;  // bytes of one 64-wide k-tile of both operands
+  // KT k-tiles per stage (one after the other): one barrier for KT tiles.
+  constexpr int kStage = KT * kSub;
+  constexpr int kSubOps = (BM + BN) / 8 / PW;  // 1 KB DMA instructions per producer wave per k-tile
+  constexpr int kOps = KT * kSubOps;           // and per stage
   static_assert(((BM + BN) / 8) % PW == 0, "DMA instructions split evenly over the producers");
   // PF: at the barrier of tile kt the producers have landed tile kt + 1 as
   // well, so the consumers read the next tile's first k-step fragments while
@@ -433,7 +436,7 @@ __global__ __launch_bounds__((CWM * CWN + PW) * 64) void linear_ring_kernel(
   }
   const int n0 = n_blk * (DUAL ? BN / 2 : BN);
   const int m0 = m_blk * BM;
-  const int ktiles = K / kBK;
+  const int ktiles = K / (kBK * KT);  // stages
 
   if (wave >= CW) {
     // ---- producers ------------------------------------------------------
@@ -454,31 +457,34 @@ __global__ __launch_bounds__((CWM * CWN + PW) * 64) void linear_ring_kernel(
     constexpr int XO = BM / 8 / PW;
     constexpr int WO = (DUAL ? BN / 2 : BN) / 8 / PW;
     static_assert(XO * PW * 8 == BM && WO * PW * 8 == (DUAL ? BN / 2 : BN) &&
-                      XO + WO * (DUAL ? 2 : 1) == kOps,
+                      XO + WO * (DUAL ? 2 : 1) == kSubOps,
                   "operands split evenly over the producers");
-    int voff[kOps];
+    int voff[kSubOps];
 #pragma unroll
-    for (int i = 0; i < kOps; ++i) {
+    for (int i = 0; i < kSubOps; ++i) {
       const int local = i < XO ? i : (i - XO) % WO;  // instruction index inside its operand
       const int row = 8 * (pw + PW * local) + lane / 8;
       const int chunk = (lane % 8) ^ (row & 7);
       voff[i] = i < XO ? static_cast<int>(row * x_rs * 2) + chunk * 16 : row * K * 2 + chunk * 16;
     }
     auto issue = [&](int kt) {
-      unsigned char* dst = ring + (kt % S) * kStage;
       const bool live = kt < ktiles;
-      const int kb = __builtin_amdgcn_readfirstlane(live ? kt * kBK * 2 : 0);
       const __amdgpu_buffer_rsrc_t lx = live ? rx : rnone;
       const __amdgpu_buffer_rsrc_t lw = live ? rw : rnone;
       const __amdgpu_buffer_rsrc_t lw2 = live ? rw2 : rnone;
 #pragma unroll
-      for (int i = 0; i < kOps; ++i) {
-        if (i < XO) {
-          lds_dma16(lx, dst + (pw + PW * i) * 1024, voff[i], kb);
-        } else if (i < XO + WO) {
-          lds_dma16(lw, dst + XB + (pw + PW * (i - XO)) * 1024, voff[i], kb);
-        } else {
-          lds_dma16(lw2, dst + XB + (BN / 2) * 128 + (pw + PW * (i - XO - WO)) * 1024, voff[i], kb);
+      for (int q = 0; q < KT; ++q) {
+        unsigned char* dst = ring + (kt % S) * kStage + q * kSub;
+        const int kb = __builtin_amdgcn_readfirstlane(live ? (kt * KT + q) * kBK * 2 : 0);
+#pragma unroll
+        for (int i = 0; i < kSubOps; ++i) {
+          if (i < XO) {
+            lds_dma16(lx, dst + (pw + PW * i) * 1024, voff[i], kb);
+          } else if (i < XO + WO) {
+            lds_dma16(lw, dst + XB + (pw + PW * (i - XO)) * 1024, voff[i], kb);
+          } else {
+            lds_dma16(lw2, dst + XB + (BN / 2) * 128 + (pw + PW * (i - XO - WO)) * 1024, voff[i], kb);
+          }
         }
       }
     };
@@ -518,19 +524,26 @@ __global__ __launch_bounds__((CWM * CWN + PW) * 64) void linear_ring_kernel(
     const unsigned char* ws = xs + XB;
     if constexpr (kPF) {
       if (kt == 0) fragments(xs, 0, na, nb);
-      typename MF::vec a[FM], b[FN];
-      fragments(xs, 1, a, b);
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+      for (int q = 0; q < KT; ++q) {
+        typename MF::vec a[FM], b[FN];
+        fragments(xs + q * kSub, 1, a, b);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = MF::run(na[i], nb[j], acc[i][j]);
-      if (kt + 1 < ktiles) fragments(ring + ((kt + 1) % S) * kStage, 0, na, nb);
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+          for (int j = 0; j < FN; ++j) acc[i][j] = MF::run(na[i], nb[j], acc[i][j]);
+        if (q + 1 < KT)
+          fragments(xs + (q + 1) * kSub, 0, na, nb);
+        else if (kt + 1 < ktiles)
+          fragments(ring + ((kt + 1) % S) * kStage, 0, na, nb);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = MF::run(a[i], b[j], acc[i][j]);
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] = MF::run(a[i], b[j], acc[i][j]);
+      }
       continue;
     }
+    static_assert(kPF || KT == 1, "several k-tiles per stage are read ahead");
 #pragma unroll
     for (int kk = 0; kk < kBK / 32; ++kk) {
       typename MF::vec a[FM], b[FN];
@@ -1039,7 +1052,7 @@ int launch_mfma(const void* x, const void* w, const void* bias, void* y, int M,
 
 // The ring kernel where the shape allows it (K a multiple of the k-tile, the
 // 16-byte store path), else the register-staged kernel of the same tile.
-template <typename T, int BM, int BN, int CWM, int CWN, int PW, int S, int GM = 8>
+template <typename T, int BM, int BN, int CWM, int CWN, int PW, int S, int GM = 8, int KT = 1>
 int launch_ring(const void* x, const void* w, const void* bias, void* y, int M, int N, int K,
                 int64_t x_rs, int64_t y_rs, hipStream_t stream, const void* residual = nullptr,
                 int64_t r_rs = 0) {
@@ -1047,9 +1060,9 @@ int launch_ring(const void* x, const void* w, const void* bias, void* y, int M, 
                    static_cast<int64_t>(BM) * y_rs * 2 < (int64_t{1} << 31) &&
                    static_cast<int64_t>(BM) * x_rs * 2 < (int64_t{1} << 31) &&
                    (residual == nullptr || static_cast<int64_t>(BM) * r_rs * 2 < (int64_t{1} << 31));
-  if (K % kBK != 0 || !vst) return kNoResidualPath;
+  if (K % (kBK * KT) != 0 || !vst) return kNoResidualPath;
   const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-  hipLaunchKernelGGL((linear_ring_kernel<T, BM, BN, CWM, CWN, PW, S, GM>), grid,
+  hipLaunchKernelGGL((linear_ring_kernel<T, BM, BN, CWM, CWN, PW, S, GM, false, false, KT>), grid,
                      dim3((CWM * CWN + PW) * 64), 0, stream, static_cast<const T*>(x),
                      static_cast<const T*>(w), static_cast<const T*>(bias), static_cast<T*>(y), M, N,
                      K, x_rs, y_rs, static_cast<const T*>(residual), r_rs);
@@ -1141,8 +1154,16 @@ int launch_ring_tile(int tile, const void* x, const void* w, const void* bias, v
         if (rc != kNoResidualPath) return rc;
       }
       return launch_ring<T, 256, 128, 4, 2, 4, 3, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s, residual, r_rs);
-    default:
+    default: {
+      // Two k-tiles per stage where K allows: with one, each barrier covers
+      // only 128 cycles of MFMAs.  M65-128 N896 K4864 17.1 -> 13.5 us (then the
+      // workgroup's own reads bound it, 93 GB/s per CU), M300-1000 18-19.2 ->
+      // 16.5-17.8, M65-500 N896 K896 6.0 -> 5.3.
+      const int rc = launch_ring<T, 64, 64, 2, 2, 2, 4, 8, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s,
+                                                             residual, r_rs);
+      if (rc != kNoResidualPath) return rc;
       return launch_ring<T, 64, 64, 2, 2, 1, 5>(x, w, bias, y, M, N, K, x_rs, y_rs, s, residual, r_rs);
+    }
   }
 }
 

@@ -153,6 +153,36 @@ def test_linear_tiles_are_bit_identical_and_exact(gpu, rows, k, n, bias):
         assert torch.equal(outputs[tile], outputs["t128x128"]), tile
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 1152])
+@pytest.mark.parametrize("rows,n", [(65, 72), (300, 896)])
+def test_linear_ring_stages_of_two_k_tiles(gpu, rows, n, k):
+    # One or two k-tiles per ring stage, fewer stages than the ring holds, and
+    # K that leaves an odd k-tile: the bits of the register-staged tile.
+    from stateful_llm_compiler_hip.backends import hip_linear
+
+    announce(f"linear r64x64 M={rows} N={n} K={k}")
+    g = generator(rows + k)
+    x = torch.randn(rows, k, generator=g).bfloat16()
+    w = (torch.randn(n, k, generator=g) * 0.02).bfloat16()
+    ring = hip_linear(x.to(gpu), w.to(gpu), tile="r64x64")
+    assert torch.equal(ring, hip_linear(x.to(gpu), w.to(gpu), tile="t64x64"))
+    assert torch.equal(ring, hip_linear(x.to(gpu), w.to(gpu)))
+    _check_linear_bf16(ring, x, w, None)
+
+
+@pytest.mark.parametrize("rows", [17, 33, 64, 65, 129, 300])
+@pytest.mark.parametrize("n,k", [(16384, 256), (16376, 128), (20001, 72)])
+def test_linear_bf16_wide_outputs_of_few_rows(gpu, rows, n, k):
+    # Either side of the vocabulary-width rule, ragged widths and K tails.
+    from stateful_llm_compiler_hip.backends import hip_linear
+
+    announce(f"linear wide M={rows} N={n} K={k}")
+    g = generator(rows + n)
+    x = torch.randn(rows, k, generator=g).bfloat16()
+    w = (torch.randn(n, k, generator=g) * 0.02).bfloat16()
+    _check_linear_bf16(hip_linear(x.to(gpu), w.to(gpu)), x, w, None, against_oracle=False)
+
+
 @pytest.mark.parametrize("rows,n", [(1000, 151936), (4096, 4864)])
 def test_linear_persistent_tile_equals_ring_tile(gpu, rows, n):
     """The persistent 256 x 128 kernel over grids many rounds deep (a
