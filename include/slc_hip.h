@@ -525,6 +525,32 @@ SLC_API int slc_hip_rope_kv_store(
     int64_t num_counters, void* stream);
 
 /*
+ * The fused projections of 33 to 64 rows (batches past the norm kernels' 32
+ * rows; the norm runs before), on the row kernel that slc_hip_linear runs such
+ * rows on, so bit for bit the single ops: up to three linears of one input,
+ * the gate/up pair with SwiGLU, the linear with its residual add (reference
+ * ops as for the entry points above).  bf16 or fp16, 16-byte aligned inputs
+ * and weights, in_features and in_stride_row multiples of 8; any features up
+ * to 16368.  SLC_ERR_UNSUPPORTED (nothing launched) otherwise.
+ */
+SLC_API int slc_hip_rows_linear_group(const void* input, int64_t in_stride_row, int64_t rows,
+                                      int64_t in_features, int count, const void* w0,
+                                      const void* b0, void* y0, int64_t n0, int64_t y0_rs,
+                                      const void* w1, const void* b1, void* y1, int64_t n1,
+                                      int64_t y1_rs, const void* w2, const void* b2, void* y2,
+                                      int64_t n2, int64_t y2_rs, int dtype, void* stream);
+SLC_API int slc_hip_rows_linear_swiglu(const void* input, int64_t in_stride_row, int64_t rows,
+                                       int64_t in_features, int64_t features, const void* w_gate,
+                                       const void* w_up, void* output, int64_t out_stride_row,
+                                       int dtype, void* stream);
+SLC_API int slc_hip_rows_linear_residual(const void* input, int64_t in_stride_row, int64_t rows,
+                                         int64_t in_features, int64_t out_features,
+                                         const void* weight, const void* bias,
+                                         const void* residual, int64_t residual_stride_row,
+                                         void* output, int64_t out_stride_row, int dtype,
+                                         void* stream);
+
+/*
  * linear_group: y_j = linear(x, w_j, b_j) for count = 1..3 matrices [n_j,
  * in_features] (the Q/K/V projections of one input) at prefill-sized rows
  * (> 64), in one launch; each output bit for bit that of slc_hip_linear

@@ -27,6 +27,7 @@ from .hip_ops import check_flag, hip_add, hip_swiglu
 from .hip_rmsnorm import hip_rms_norm
 
 MAX_FUSED_ROWS = 32
+MAX_PLAIN_ROWS = 64  # rows the row kernel takes without a norm
 _UNSUPPORTED = -2  # SLC_ERR_UNSUPPORTED
 _MATRICES = 3
 
@@ -166,7 +167,9 @@ def _linear_group(x: torch.Tensor, weights: Sequence[torch.Tensor],
                            outputs[i].data_ptr(), weights[i].shape[0], weights[i].shape[0]]
         else:
             per_matrix += [None, None, None, 0, 0]
-    status = _native.library().slc_hip_linear_group(
+    lib = _native.library()
+    entry = lib.slc_hip_rows_linear_group if rows <= MAX_PLAIN_ROWS else lib.slc_hip_linear_group
+    status = entry(
         x.data_ptr(), hidden, rows, hidden, len(weights), *per_matrix,
         _native.dtype_tag(x.dtype), _native.current_stream(x.device),
     )
@@ -188,7 +191,9 @@ def _linear_swiglu(x: torch.Tensor, gate_weight: torch.Tensor,
         return None
     features = gate_weight.shape[0]
     out = torch.empty((*x.shape[:-1], features), device=x.device, dtype=x.dtype)
-    status = _native.library().slc_hip_linear_swiglu(
+    lib = _native.library()
+    entry = lib.slc_hip_rows_linear_swiglu if rows <= MAX_PLAIN_ROWS else lib.slc_hip_linear_swiglu
+    status = entry(
         x.data_ptr(), hidden, rows, hidden, features, gate_weight.data_ptr(),
         up_weight.data_ptr(), out.data_ptr(), features, _native.dtype_tag(x.dtype),
         _native.current_stream(x.device),
@@ -216,8 +221,9 @@ def hip_linear_residual(
         raise ValueError("HIP linear_residual: residual and bias must be on the GPU")
     hidden = tensor.shape[-1]
     rows = tensor.numel() // hidden if hidden else 0
-    # Decode-sized rows take the fused row kernel; prefill-sized rows the tile
-    # kernel with the residual in its store epilogue, when it takes the shape.
+    # Decode-sized rows (up to 64) take the fused row kernel; prefill-sized rows
+    # the tile kernel with the residual in its store epilogue, when it takes the
+    # shape.
     prefill = (rows > MAX_FUSED_ROWS and tensor.is_cuda and tensor.is_contiguous()
                and residual.is_contiguous() and tensor.dtype in (torch.bfloat16, torch.float16)
                and (bias is None or (bias.dtype == tensor.dtype and bias.is_contiguous())))
@@ -225,7 +231,10 @@ def hip_linear_residual(
         return hip_add(residual, hip_linear(tensor, weight, bias))
     features = weight.shape[0]
     out = torch.empty(out_shape, device=tensor.device, dtype=tensor.dtype)
-    status = _native.library().slc_hip_linear_residual(
+    lib = _native.library()
+    entry = (lib.slc_hip_rows_linear_residual if MAX_FUSED_ROWS < rows <= MAX_PLAIN_ROWS
+             else lib.slc_hip_linear_residual)
+    status = entry(
         tensor.data_ptr(), hidden, tensor.numel() // hidden, hidden, features,
         weight.data_ptr(), None if bias is None else bias.data_ptr(), residual.data_ptr(),
         features, out.data_ptr(), features, _native.dtype_tag(tensor.dtype),

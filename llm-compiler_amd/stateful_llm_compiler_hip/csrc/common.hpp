@@ -197,12 +197,6 @@ int decode_attention_f32(const float* query, const float* kb, const float* vb, c
                          const int64_t* strides, float scale, hipStream_t stream);
 bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                           int dtype);
-int rows_group(const void* x, int64_t x_rs, int64_t rows, int64_t K, int count,
-               const void* const* w, const void* const* bias, void* const* y, const int64_t* n,
-               const int64_t* y_rs, int dtype, hipStream_t stream);
-int rows_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
-                const void* w_gate, const void* w_up, void* y, int64_t y_rs, int dtype,
-                hipStream_t stream);
 int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                 const void* w, const void* bias, void* y, int64_t y_rs, int dtype,
                 hipStream_t stream);

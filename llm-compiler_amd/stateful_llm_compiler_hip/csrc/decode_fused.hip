@@ -22,6 +22,8 @@
 // Semantics: src/stateful_llm_compiler/execution.py:674-692 (rms_norm),
 // triton_executor.py:159-176 (linear), :741-767 (rope), :743-781 (kv store).
 
+#include <initializer_list>
+
 #include "common.hpp"
 #include "op_math.hpp"
 
@@ -765,74 +767,6 @@ bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, 
          N <= (1 << 24) && (rows <= 16 || (N + 15) / 16 < kWideBlocks);
 }
 
-// The fused forms for 33 .. 64 rows (their norm, if any, ran before): up to
-// three linears of one input, the SwiGLU pair, the linear with its residual
-// add.  SLC_ERR_UNSUPPORTED (nothing launched) for shapes they do not take.
-int rows_group(const void* x, int64_t x_rs, int64_t rows, int64_t K, int count,
-               const void* const* w, const void* const* bias, void* const* y, const int64_t* n,
-               const int64_t* y_rs, int dtype, hipStream_t stream) {
-  FusedArgs a{};
-  a.x = x;
-  a.x_rs = x_rs;
-  a.rows = static_cast<int>(rows);
-  a.hidden = static_cast<int>(K);
-  for (int i = 0; i < count; ++i) {
-    if (w[i] == nullptr || y[i] == nullptr || n[i] < 1 || y_rs[i] < n[i] ||
-        (reinterpret_cast<uintptr_t>(w[i]) & 15) != 0 ||
-        !rows_linear_eligible(x, x_rs, rows, K, n[i], dtype))
-      return SLC_ERR_UNSUPPORTED;
-    a.w[i] = w[i];
-    a.bias[i] = bias[i];
-    a.y[i] = y[i];
-    a.n[i] = static_cast<int>(n[i]);
-    a.y_rs[i] = y_rs[i];
-  }
-  assign_blocks(a, count);
-  return dispatch_rows<kStore>(a, dtype, stream);
-}
-
-int rows_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
-                const void* w_gate, const void* w_up, void* y, int64_t y_rs, int dtype,
-                hipStream_t stream) {
-  const uint64_t bits = reinterpret_cast<uintptr_t>(w_gate) | reinterpret_cast<uintptr_t>(w_up);
-  if ((bits & 15) != 0 || y_rs < N || !rows_linear_eligible(x, x_rs, rows, K, N, dtype))
-    return SLC_ERR_UNSUPPORTED;
-  FusedArgs a{};
-  a.x = x;
-  a.x_rs = x_rs;
-  a.rows = static_cast<int>(rows);
-  a.hidden = static_cast<int>(K);
-  a.w[0] = w_gate;
-  a.w[1] = w_up;
-  a.y[0] = y;
-  a.n[0] = static_cast<int>(N);
-  a.y_rs[0] = y_rs;
-  assign_blocks(a, 1);
-  return dispatch_rows<kSwiglu>(a, dtype, stream);
-}
-
-int rows_residual(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N, const void* w,
-                  const void* bias, const void* residual, int64_t r_rs, void* y, int64_t y_rs,
-                  int dtype, hipStream_t stream) {
-  if ((reinterpret_cast<uintptr_t>(w) & 15) != 0 || y_rs < N || r_rs < N ||
-      !rows_linear_eligible(x, x_rs, rows, K, N, dtype))
-    return SLC_ERR_UNSUPPORTED;
-  FusedArgs a{};
-  a.x = x;
-  a.x_rs = x_rs;
-  a.rows = static_cast<int>(rows);
-  a.hidden = static_cast<int>(K);
-  a.w[0] = w;
-  a.bias[0] = bias;
-  a.y[0] = y;
-  a.n[0] = static_cast<int>(N);
-  a.y_rs[0] = y_rs;
-  a.residual = residual;
-  a.r_rs = r_rs;
-  assign_blocks(a, 1);
-  return dispatch_rows<kResidual>(a, dtype, stream);
-}
-
 }  // namespace slc_host
 
 extern "C" int slc_hip_norm_linear_group(
@@ -915,10 +849,6 @@ extern "C" int slc_hip_linear_residual(const void* x, int64_t x_rs, int64_t rows
     // Prefill-sized: the tile kernel with the residual in its store epilogue.
     SLC_REQUIRE(x && weight && residual && y && in_features >= 1 && out_features >= 1,
                 "%s: bad operands", what);
-    if (rows <= kMaxPlainRows)
-      return slc_host::rows_residual(x, x_rs, rows, in_features, out_features, weight, bias,
-                                     residual, residual_rs, y, y_rs, dtype,
-                                     static_cast<hipStream_t>(stream));
     return slc_host::gemm_residual(x, x_rs, rows, in_features, out_features, weight, bias,
                                    residual, residual_rs, y, y_rs, dtype,
                                    static_cast<hipStream_t>(stream));
@@ -939,6 +869,101 @@ extern "C" int slc_hip_linear_residual(const void* x, int64_t x_rs, int64_t rows
   a.y_rs[0] = y_rs;
   a.residual = residual;
   a.r_rs = residual_rs;
+  assign_blocks(a, 1);
+  return dispatch_rows<kResidual>(a, dtype, static_cast<hipStream_t>(stream));
+}
+
+// ---- 33 to 64 rows ----------------------------------------------------------
+// The fused forms without their norm (it ran before): up to three linears of
+// one input, the SwiGLU pair, the linear with its residual add.
+
+namespace {
+
+// Whether the row kernel takes these rows and this weight; nothing is
+// launched otherwise.
+bool plain_rows_ok(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N, const void* w,
+                   const void* y, int64_t y_rs, int dtype) {
+  return rows > kMaxRows && x != nullptr && w != nullptr && y != nullptr && x_rs >= K && N >= 1 &&
+         y_rs >= N && (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
+         slc_host::rows_linear_eligible(x, x_rs, rows, K, N, dtype);
+}
+FusedArgs plain_rows(const void* x, int64_t x_rs, int64_t rows, int64_t K) {
+  FusedArgs a{};
+  a.x = x;
+  a.x_rs = x_rs;
+  a.rows = static_cast<int>(rows);
+  a.hidden = static_cast<int>(K);
+  return a;
+}
+
+}  // namespace
+
+extern "C" int slc_hip_rows_linear_group(const void* input, int64_t in_stride_row, int64_t rows,
+                                         int64_t in_features, int count, const void* w0,
+                                         const void* b0, void* y0, int64_t n0, int64_t y0_rs,
+                                         const void* w1, const void* b1, void* y1, int64_t n1,
+                                         int64_t y1_rs, const void* w2, const void* b2, void* y2,
+                                         int64_t n2, int64_t y2_rs, int dtype, void* stream) {
+  SLC_REQUIRE(rows >= 0 && in_features > 0 && count >= 1 && count <= kMaxMatrices,
+              "slc_hip_rows_linear_group: bad sizes");
+  const void* ws[3] = {w0, w1, w2};
+  const void* bs[3] = {b0, b1, b2};
+  void* ys[3] = {y0, y1, y2};
+  const int64_t ns[3] = {n0, n1, n2};
+  const int64_t rss[3] = {y0_rs, y1_rs, y2_rs};
+  FusedArgs a = plain_rows(input, in_stride_row, rows, in_features);
+  for (int i = 0; i < count; ++i) {
+    if (!plain_rows_ok(input, in_stride_row, rows, in_features, ns[i], ws[i], ys[i], rss[i], dtype))
+      return SLC_ERR_UNSUPPORTED;
+    a.w[i] = ws[i];
+    a.bias[i] = bs[i];
+    a.y[i] = ys[i];
+    a.n[i] = static_cast<int>(ns[i]);
+    a.y_rs[i] = rss[i];
+  }
+  assign_blocks(a, count);
+  return dispatch_rows<kStore>(a, dtype, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int slc_hip_rows_linear_swiglu(const void* input, int64_t in_stride_row, int64_t rows,
+                                          int64_t in_features, int64_t features,
+                                          const void* w_gate, const void* w_up, void* output,
+                                          int64_t out_stride_row, int dtype, void* stream) {
+  SLC_REQUIRE(rows >= 0 && in_features > 0 && features > 0, "slc_hip_rows_linear_swiglu: bad sizes");
+  for (const void* w : {w_gate, w_up})
+    if (!plain_rows_ok(input, in_stride_row, rows, in_features, features, w, output, out_stride_row,
+                       dtype))
+      return SLC_ERR_UNSUPPORTED;
+  FusedArgs a = plain_rows(input, in_stride_row, rows, in_features);
+  a.w[0] = w_gate;
+  a.w[1] = w_up;
+  a.y[0] = output;
+  a.n[0] = static_cast<int>(features);
+  a.y_rs[0] = out_stride_row;
+  assign_blocks(a, 1);
+  return dispatch_rows<kSwiglu>(a, dtype, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int slc_hip_rows_linear_residual(const void* input, int64_t in_stride_row, int64_t rows,
+                                            int64_t in_features, int64_t out_features,
+                                            const void* weight, const void* bias,
+                                            const void* residual, int64_t residual_stride_row,
+                                            void* output, int64_t out_stride_row, int dtype,
+                                            void* stream) {
+  SLC_REQUIRE(rows >= 0 && in_features > 0 && out_features > 0,
+              "slc_hip_rows_linear_residual: bad sizes");
+  if (residual == nullptr || residual_stride_row < out_features ||
+      !plain_rows_ok(input, in_stride_row, rows, in_features, out_features, weight, output,
+                     out_stride_row, dtype))
+    return SLC_ERR_UNSUPPORTED;
+  FusedArgs a = plain_rows(input, in_stride_row, rows, in_features);
+  a.w[0] = weight;
+  a.bias[0] = bias;
+  a.y[0] = output;
+  a.n[0] = static_cast<int>(out_features);
+  a.y_rs[0] = out_stride_row;
+  a.residual = residual;
+  a.r_rs = residual_stride_row;
   assign_blocks(a, 1);
   return dispatch_rows<kResidual>(a, dtype, static_cast<hipStream_t>(stream));
 }

@@ -1262,8 +1262,6 @@ int gemm_residual(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t 
 int gemm_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                 const void* w_gate, const void* w_up, void* y, int64_t y_rs, int dtype,
                 hipStream_t stream) {
-  if (rows > 32 && rows <= 64)
-    return rows_swiglu(x, x_rs, rows, K, N, w_gate, w_up, y, y_rs, dtype, stream);
   const uint64_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w_gate) |
                         reinterpret_cast<uintptr_t>(w_up) | reinterpret_cast<uintptr_t>(y);
   const bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 64 && (bits & 15) == 0 &&
@@ -1306,8 +1304,6 @@ int gemm_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
 int gemm_group(const void* x, int64_t x_rs, int64_t rows, int64_t K, int count,
                const void* const* w, const void* const* bias, void* const* y,
                const int64_t* n, const int64_t* y_rs, int dtype, hipStream_t stream) {
-  if (rows > 32 && rows <= 64)
-    return rows_group(x, x_rs, rows, K, count, w, bias, y, n, y_rs, dtype, stream);
   bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 64 && count >= 1 && count <= 3 &&
             K % kBK == 0 && x_rs % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
             128 * x_rs * 2 < (int64_t{1} << 31) && rows < (int64_t{1} << 31);

@@ -115,6 +115,29 @@ def test_fused_entry_points_decline_or_reject_before_any_device_call():
     assert lib.slc_hip_rope_decode_attention(*args, bf16, *sizes, *strides, 0.125, 7, None) == -1
 
 
+def test_row_kernel_entry_points_decline_other_rows():
+    # 33 to 64 rows, K a multiple of 8, widths below the vocabulary kernels',
+    # 16-byte aligned weights; everything else is declined before a launch.
+    lib = _native.library()
+    p, bf16, f32 = 0x1000, 2, 0
+
+    def group(rows=40, k=896, n=128, w=p, dtype=bf16):
+        return lib.slc_hip_rows_linear_group(p, k, rows, k, 1, w, None, p, n, n, None, None, None, 0, 0,
+                                             None, None, None, 0, 0, dtype, None)
+
+    def swiglu(rows=40, k=896, n=128, w=p, dtype=bf16):
+        return lib.slc_hip_rows_linear_swiglu(p, k, rows, k, n, p, w, p, n, dtype, None)
+
+    def residual(rows=40, k=896, n=128, w=p, dtype=bf16):
+        return lib.slc_hip_rows_linear_residual(p, k, rows, k, n, w, None, p, n, p, n, dtype, None)
+
+    for call in (group, swiglu, residual):
+        for bad in ({"rows": 32}, {"rows": 65}, {"rows": 0}, {"k": 900}, {"n": 20000}, {"w": p + 8}, {"w": None},
+                    {"dtype": f32}):
+            assert call(**bad) == -2, (call.__name__, bad)
+        assert call(k=0) == -1
+
+
 def test_paged_kv_store_rejects_a_grid_past_one_launch():
     # 2^43 16-byte units need 2^35 workgroups of 256, past a launch: rejected on
     # the host (the pointers are never dereferenced).
