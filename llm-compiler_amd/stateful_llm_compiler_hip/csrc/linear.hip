@@ -683,6 +683,10 @@ __device__ __forceinline__ void xcd_tile_of(int id, int n_tiles, int m_tiles, in
 // DUAL: each 128-row W stage holds 64 gate rows then 64 up rows; consumer
 // wave wn takes gate and up rows of the same 32 features (fragments 0-1 gate,
 // 2-3 up), so the SwiGLU pairs meet in one lane.
+// The W tile's own swizzle: the 16 rows of a fragment read below are four runs
+// of four, eight apart, so the key takes row bits 0, 1 and 3.
+__device__ __forceinline__ int w_key(int row) { return (row & 3) | ((row >> 1) & 4); }
+
 template <typename T, bool DUAL>
 __global__ __launch_bounds__(12 * 64) void linear_stream_kernel(
     const T* __restrict__ x, const T* __restrict__ w_arg, const T* __restrict__ bias_arg,
@@ -734,7 +738,7 @@ __global__ __launch_bounds__(12 * 64) void linear_stream_kernel(
     for (int i = 0; i < kOps; ++i) {
       const int local = i < XO ? i : (i - XO) % WO;
       const int row = 8 * (pw + PW * local) + lane / 8;
-      const int chunk = (lane % 8) ^ (row & 7);
+      const int chunk = (lane % 8) ^ (i < XO ? row & 7 : w_key(row));
       voff[i] = i < XO ? static_cast<int>(row * x_rs * 2) + chunk * 16 : row * K * 2 + chunk * 16;
     }
     // The operand ranges of the tile being loaded, as base + bytes: the
@@ -810,7 +814,7 @@ __global__ __launch_bounds__(12 * 64) void linear_stream_kernel(
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
       braw[j][0] = braw[j][1] = 0u;
-      const int n = t.n0 + wn * TN + j * 16 + 4 * g;
+      const int n = t.n0 + wn * TN + (j >> 1) * 32 + 8 * g + (j & 1) * 4;
       if (!DUAL && t.bias != nullptr && n < t.N) {
         const uint16_t* bp = reinterpret_cast<const uint16_t*>(t.bias + n);
         braw[j][0] = bp[0] | (static_cast<uint32_t>(bp[1]) << 16);
@@ -837,9 +841,13 @@ __global__ __launch_bounds__(12 * 64) void linear_stream_kernel(
           a[i] = *reinterpret_cast<const typename MF::vec*>(xs + lds_offset(wm * TM + i * 16 + c, kk * 4 + g));
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          const int wrow = DUAL ? (j < 2 ? wn * 32 + j * 16 : BN / 2 + wn * 32 + (j - 2) * 16)
-                                : wn * TN + j * 16;
-          b[j] = *reinterpret_cast<const typename MF::vec*>(ws + lds_offset(wrow + c, kk * 4 + g));
+          // Fragment row c is feature 8 (c / 4) + c % 4 (+ 4 in odd fragments)
+          // of a run of 32, so that a lane's two fragments of the run hold
+          // eight consecutive features.
+          const int wrow = (DUAL ? (j < 2 ? wn * 32 : BN / 2 + wn * 32) : wn * TN + (j >> 1) * 32) +
+                           8 * (c >> 2) + (j & 1) * 4 + (c & 3);
+          b[j] = *reinterpret_cast<const typename MF::vec*>(
+              ws + wrow * (kBK * 2) + (((kk * 4 + g) ^ w_key(wrow)) << 4));
         }
 #pragma unroll
         for (int j = 0; j < FN; ++j)
@@ -847,36 +855,41 @@ __global__ __launch_bounds__(12 * 64) void linear_stream_kernel(
           for (int i = 0; i < FM; ++i) acc[j][i] = MF::run(b[j], a[i], acc[j][i]);
       }
     }
-    // Epilogue: lane (c, g) of fragment (j, i) holds features 4g .. 4g + 3 of
-    // row c.
+    // Epilogue: lane (c, g) of fragments (2p, i) and (2p + 1, i) holds features
+    // 8g .. 8g + 7 of run p of row c: one 16-byte store, 64 bytes of a row by
+    // its four lanes.  (With four features per lane the 8-byte stores took
+    // 468 of 1316 us at the vocabulary head, timed against a copy without
+    // them, and 78 of 343 at M32768 N4864.)
     const int rows = M - t.m0 < BM ? M - t.m0 : BM;
     const __amdgpu_buffer_rsrc_t ry =
         make_rsrc(t.y + t.m0 * t.y_rs, (static_cast<int64_t>(rows) - 1) * t.y_rs * 2 + t.N * 2);
-    constexpr int kOutFrags = DUAL ? FN / 2 : FN;
+    constexpr int kRuns = DUAL ? 1 : 2;
 #pragma unroll
-    for (int j = 0; j < kOutFrags; ++j) {
-      const int n = t.n0 + (DUAL ? wn * 32 : wn * TN) + j * 16 + 4 * g;
+    for (int p = 0; p < kRuns; ++p) {
+      const int n = t.n0 + (DUAL ? wn * 32 : wn * TN + p * 32) + 8 * g;
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
         const int m_local = wm * TM + i * 16 + c;
-        uint16_t o[4];
+        uint32_t o[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int e = 0; e < 8; ++e) {
+          const int j = 2 * p + (e >> 2), r = e & 3;
           if constexpr (DUAL) {
             const T ge = slc::from_f32<T>(acc[j][i][r]);
             const T ue = slc::from_f32<T>(acc[j + 2][i][r]);
-            o[r] = slc::from_f32<T>(slc::swiglu_value<T>(slc::to_f32(ge), slc::to_f32(ue))).bits;
+            o[e] = slc::from_f32<T>(slc::swiglu_value<T>(slc::to_f32(ge), slc::to_f32(ue))).bits;
           } else {
             T bt;
             bt.bits = static_cast<uint16_t>(braw[j][r >> 1] >> (16 * (r & 1)));
-            o[r] = slc::from_f32<T>(acc[j][i][r] + slc::to_f32(bt)).bits;
+            o[e] = slc::from_f32<T>(acc[j][i][r] + slc::to_f32(bt)).bits;
           }
         }
         if (m_local < rows && n < t.N) {
-          const uint2 packed = make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16),
-                                          o[2] | (static_cast<uint32_t>(o[3]) << 16));
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2_t, packed), ry,
-                                                static_cast<int>(m_local * t.y_rs + n) * 2, 0, 0);
+          i32x4_t packed;
+#pragma unroll
+          for (int d = 0; d < 4; ++d) packed[d] = static_cast<int>(o[2 * d] | (o[2 * d + 1] << 16));
+          __builtin_amdgcn_raw_buffer_store_b128(packed, ry,
+                                                 static_cast<int>(m_local * t.y_rs + n) * 2, 0, 0);
         }
       }
     }
@@ -1076,9 +1089,10 @@ int launch_ring(const void* x, const void* w, const void* bias, void* y, int M, 
 // The persistent 256 x 128 form (linear_stream_kernel): one workgroup per CU
 // (a multiple of 8, so each one's tiles stay on its XCD), or one per tile
 // when there are fewer tiles.  kNoResidualPath where the shape does not fit.
-// The library launches it for gate/up + SwiGLU (4-9 % faster there than the
-// ring kernel, whose SwiGLU epilogue stages the whole tile in LDS); for plain
-// linears it times within 2 % of the ring kernel and is a plan's choice.
+// The library launches it for plain linears and gate/up + SwiGLU from two rounds
+// of tiles on: its stores drain under the next tile's MFMAs, where the ring
+// kernel's workgroups end with them (M4096 N4864 K896 43.9 -> 40.1 us, M8192
+// 73.9 -> 66.3, M32768 341 -> 308, vocabulary head of 4096 rows 1270 -> 1202).
 template <typename T, bool DUAL>
 int launch_stream(const void* x, const void* w, const void* bias, void* y, int M, int N, int K,
                   int64_t x_rs, int64_t y_rs, int n_tiles, hipStream_t stream,
@@ -1184,8 +1198,12 @@ int dispatch_mfma(const void* x, const void* w, const void* bias, void* y, int M
   // Tile variants (a profile plan picks one): every tile accumulates each
   // output's k range in the same order, 32 k at a time on one MFMA chain, so
   // the variants differ in speed only, never in a bit of the result.
-  if (tile == SLC_TILE_AUTO)
+  if (tile == SLC_TILE_AUTO) {
     tile = wide_on_register_tiles(M, N) ? SLC_TILE_128X128 : auto_ring_tile(M, (N + 127) / 128);
+    // Two rounds of 256 x 128 tiles or more: the persistent form.
+    if (tile == SLC_TILE_R256X128 && stream_grid(int64_t{(M + 255) / 256} * ((N + 127) / 128)))
+      tile = SLC_TILE_S256X128;
+  }
   switch (tile) {
     case SLC_TILE_128X64:
       return launch_mfma<T, 128, 64, 2, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
