@@ -375,14 +375,33 @@ int dispatch_v2(const void* q, const void* k, const void* v, const void* mask, i
   // T1024: 64.6 -> 58.3; at T4096 the 32-query form is 8 % faster.
   const int64_t grid32 = int64_t{kv_heads} * batch * ((tokens + 31) / 32);
   const bool short_grid = grid32 <= int64_t{SLC_PREFILL_SHORT_ROUNDS} * slc_host::device_cu_count();
+  // Seven or eight heads in one workgroup put two waves on every SIMD, and a
+  // short grid is bound by its longest workgroup's chain of key tiles, so there
+  // the group is split over workgroups of four heads (twice the grid, K and V
+  // read twice): while the 16-query grid is at most one and a half workgroups
+  // per CU (B3 T1000 fp16 exact with a mask 34.9 -> 27.9 us, B4 T512 18.3 ->
+  // 15.7, B1 T1000 online 13.6 -> 10.5), or two where sequences are long enough
+  // for the causal imbalance to matter (B1 T4096 57.7 -> 51.3, B2 T2048 exact
+  // 46.2 -> 41.8).  Deeper grids keep the whole group: B8 T512 20.4 us, split
+  // 24.4; B8 T800 37.5, split 49.2.
+  constexpr int GW = G >= 7 ? 4 : G;
+  const int64_t grid16 = int64_t{kv_heads} * batch * ((tokens + 15) / 16);
+  const int64_t cus = slc_host::device_cu_count();
+  const bool split = GW != G && (2 * grid16 <= 3 * cus || (grid16 <= 2 * cus && tokens >= 1024));
   // One braced statement: each use below sits under an if.
+#define SLC_SHORT(W, MKV)                                                                            \
+  return causal ? slc_prefill::launch_v2_short<T, W, MKV, true>(q, k, v, mask, out, batch, tokens,    \
+                                                                kv_heads, st, scale, exact, classes, s, G) \
+                : slc_prefill::launch_v2_short<T, W, MKV, false>(q, k, v, mask, out, batch, tokens,   \
+                                                                 kv_heads, st, scale, exact, classes, s, G)
 #define SLC_V2(MKV)                                                                                  \
   {                                                                                                   \
-    if (short_grid)                                                                                   \
-      return causal ? slc_prefill::launch_v2_short<T, G, MKV, true>(q, k, v, mask, out, batch, tokens, \
-                                                                    kv_heads, st, scale, exact, classes, s) \
-                    : slc_prefill::launch_v2_short<T, G, MKV, false>(q, k, v, mask, out, batch, tokens, \
-                                                                     kv_heads, st, scale, exact, classes, s); \
+    if (short_grid && split) {                                                                        \
+      SLC_SHORT(GW, MKV);                                                                             \
+    }                                                                                                 \
+    if (short_grid) {                                                                                 \
+      SLC_SHORT(G, MKV);                                                                              \
+    }                                                                                                 \
     return causal ? launch_v2<T, G, MKV, true, 2>(q, k, v, mask, out, batch, tokens, kv_heads, st, scale, exact, classes, s) \
                   : launch_v2<T, G, MKV, false, 2>(q, k, v, mask, out, batch, tokens, kv_heads, st, scale, exact, classes, s); \
   }
@@ -391,6 +410,7 @@ int dispatch_v2(const void* q, const void* k, const void* v, const void* mask, i
   if (mask_dtype == SLC_F16) SLC_V2(SLC_F16 + 1)
   SLC_V2(SLC_F32 + 1)
 #undef SLC_V2
+#undef SLC_SHORT
 }
 
 template <typename T>

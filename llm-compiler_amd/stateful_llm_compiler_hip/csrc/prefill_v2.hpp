@@ -158,7 +158,7 @@ __global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attenti
     int64_t q_sb, int64_t q_sh, int64_t q_st, int64_t k_sb, int64_t k_sh, int64_t k_st,
     int64_t v_sb, int64_t v_sh, int64_t v_st, int64_t m_sb, int64_t m_sq, int64_t o_sb,
     int64_t o_sh, int64_t o_st, float scale, const unsigned char* __restrict__ tile_class,
-    int m_step) {
+    int m_step, int group, int splits) {
   using M = Mfma<T>;
   constexpr int kQB = QB;                // query blocks of 16 per consumer wave
   constexpr int kV2Queries = 16 * QB;    // queries per workgroup
@@ -178,7 +178,10 @@ __global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attenti
   // scheduling.  Any other shape is indifferent to the order.
   const int nqb = gridDim.z;
   const int qblk = nqb - 1 - static_cast<int>(blockIdx.z);
-  const int kvh = blockIdx.x;
+  // The KV head's group of query heads may be split over several workgroups of
+  // G heads each (the last one's spare waves only meet the barriers).
+  const int kvh = blockIdx.x / splits;
+  const int head0 = (blockIdx.x % splits) * G;
   const int64_t b = blockIdx.y;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -327,8 +330,12 @@ __global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attenti
     return;
   }
 
-  // ---- consumers: wave w computes query head kvh * G + w ----------------------
-  const int h = kvh * G + wave;
+  // ---- consumers: one query head per wave -------------------------------------
+  if (head0 + wave >= group) {
+    for (int step = 0; step < nsteps; ++step) __syncthreads();
+    return;
+  }
+  const int h = kvh * group + head0 + wave;
   typename M::vec qv[kQB][2];
 #pragma unroll
   for (int qb = 0; qb < kQB; ++qb) {
@@ -634,8 +641,9 @@ inline int mask_step(const void* mask, const int64_t* st, int tokens, int es) {
 template <typename T, int G, int MK, bool CAUSAL, int QB>
 int launch_v2(const void* q, const void* k, const void* v, const void* mask, void* out,
               int64_t batch, int tokens, int kv_heads, const int64_t* st, float scale,
-              bool exact, const unsigned char* classes, hipStream_t stream) {
-  const dim3 grid(kv_heads, static_cast<unsigned>(batch), (tokens + 16 * QB - 1) / (16 * QB));
+              bool exact, const unsigned char* classes, hipStream_t stream, int group = G) {
+  const int splits = (group + G - 1) / G;
+  const dim3 grid(kv_heads * splits, static_cast<unsigned>(batch), (tokens + 16 * QB - 1) / (16 * QB));
   int exponent = 0;
   const bool pow2 = std::is_same_v<T, slc::bf16_t> && std::frexp(scale, &exponent) == 0.5f &&
                     exponent > -100;
@@ -648,7 +656,7 @@ int launch_v2(const void* q, const void* k, const void* v, const void* mask, voi
                      static_cast<const T*>(v), mask, static_cast<T*>(out), tokens, kv_heads,
                      st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7], st[8], st[9], st[10],
                      st[12], st[13], st[14], scale, MK != 0 ? classes : nullptr,
-                     MK != 0 ? mask_step(mask, st, tokens, mask_elem_bytes<MK>()) : 0);
+                     MK != 0 ? mask_step(mask, st, tokens, mask_elem_bytes<MK>()) : 0, group, splits);
   return slc_host::check_launch("slc_hip_prefill_attention(grouped)");
 }
 
@@ -660,5 +668,5 @@ namespace slc_prefill {
 template <typename T, int G, int MK, bool CAUSAL>
 int launch_v2_short(const void* q, const void* k, const void* v, const void* mask, void* out,
                     int64_t batch, int tokens, int kv_heads, const int64_t* st, float scale,
-                    bool exact, const unsigned char* classes, hipStream_t stream);
+                    bool exact, const unsigned char* classes, hipStream_t stream, int group);
 }  // namespace slc_prefill

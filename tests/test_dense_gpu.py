@@ -770,3 +770,39 @@ def test_prefill_masks_in_any_layout_agree(gpu, tokens, layout, order, mask_dtyp
     torch.cuda.synchronize()
     assert torch.equal(actual.view(torch.int16), wanted.view(torch.int16))
     assert_bf16_close(actual.cpu(), ref.prefill_attention(q, k, v, values, groups=7, scale=0.125, causal=False))
+
+
+@pytest.mark.parametrize("q_heads,kv_heads", [(14, 2), (16, 2)])
+@pytest.mark.parametrize("batch,tokens,kind", [(12, 256, "causal-online"), (12, 250, "mask-exact"),
+                                               (3, 1366, "causal-exact"), (1, 5, "mask-online")])
+def test_prefill_split_head_groups_agree(gpu, q_heads, kv_heads, batch, tokens, kind):
+    """Short grids split a group of seven or eight heads over workgroups of
+    four; batch rows are independent, so a batch whose grid keeps the group
+    whole gives the same bits for the rows of a batch whose grid does not."""
+
+    from stateful_llm_compiler_hip.backends import hip_prefill_attention
+
+    announce(f"prefill split head groups B={batch} T={tokens} QH={q_heads} {kind}")
+    g = torch.Generator(device=gpu).manual_seed(tokens)
+    repeat = -(-600 * 16 // (kv_heads * batch * tokens))  # past two workgroups per CU
+    q, k, v = (torch.randn(batch, h, tokens, 64, device=gpu, generator=g, dtype=torch.bfloat16)
+               for h in (q_heads, kv_heads, kv_heads))
+    structure, order = kind.split("-")
+    mask = None
+    if structure == "mask":
+        future = torch.ones(tokens, tokens, dtype=torch.bool, device=gpu).triu(1)
+        mask = torch.zeros(batch, 1, tokens, tokens, device=gpu).masked_fill(future, float("-inf"))
+
+    def run(times):
+        def many(t):
+            return None if t is None else t.repeat(times, 1, 1, 1)
+
+        return hip_prefill_attention(many(q), many(k), many(v), many(mask), scale=0.125,
+                                     causal=structure == "causal", softmax_order=order)[:batch]
+
+    short, deep = run(1), run(repeat)
+    torch.cuda.synchronize()
+    assert torch.equal(short.view(torch.int16), deep.view(torch.int16))
+    expected = ref.prefill_attention(q.cpu(), k.cpu(), v.cpu(), None if mask is None else mask.cpu(),
+                                     groups=q_heads // kv_heads, scale=0.125, causal=structure == "causal")
+    assert_bf16_close(short.cpu(), expected)
