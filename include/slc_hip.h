@@ -526,12 +526,14 @@ SLC_API int slc_hip_rope_kv_store(
 
 /*
  * The fused projections of 33 to 64 rows (batches past the norm kernels' 32
- * rows; the norm runs before), on the row kernel that slc_hip_linear runs such
+ * rows; the norm runs before), on the kernels that slc_hip_linear runs such
  * rows on, so bit for bit the single ops: up to three linears of one input,
  * the gate/up pair with SwiGLU, the linear with its residual add (reference
  * ops as for the entry points above).  bf16 or fp16, 16-byte aligned inputs
- * and weights, in_features and in_stride_row multiples of 8; any features up
- * to 16368.  SLC_ERR_UNSUPPORTED (nothing launched) otherwise.
+ * and weights, in_features and in_stride_row multiples of 8; features up to
+ * 16368; from 4096 features on also 16-byte aligned outputs, in_features a
+ * multiple of 64, features and all strides multiples of 8.
+ * SLC_ERR_UNSUPPORTED (nothing launched) otherwise.
  */
 SLC_API int slc_hip_rows_linear_group(const void* input, int64_t in_stride_row, int64_t rows,
                                       int64_t in_features, int count, const void* w0,

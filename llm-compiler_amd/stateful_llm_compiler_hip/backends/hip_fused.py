@@ -27,7 +27,7 @@ from .hip_ops import check_flag, hip_add, hip_swiglu
 from .hip_rmsnorm import hip_rms_norm
 
 MAX_FUSED_ROWS = 32
-MAX_PLAIN_ROWS = 64  # rows the row kernel takes without a norm
+MAX_PLAIN_ROWS = 64  # rows that have fused forms without a norm of their own
 _UNSUPPORTED = -2  # SLC_ERR_UNSUPPORTED
 _MATRICES = 3
 
@@ -221,9 +221,8 @@ def hip_linear_residual(
         raise ValueError("HIP linear_residual: residual and bias must be on the GPU")
     hidden = tensor.shape[-1]
     rows = tensor.numel() // hidden if hidden else 0
-    # Decode-sized rows (up to 64) take the fused row kernel; prefill-sized rows
-    # the tile kernel with the residual in its store epilogue, when it takes the
-    # shape.
+    # Decode-sized rows take the fused row kernel; more rows the tile kernel
+    # with the residual in its store epilogue, when it takes the shape.
     prefill = (rows > MAX_FUSED_ROWS and tensor.is_cuda and tensor.is_contiguous()
                and residual.is_contiguous() and tensor.dtype in (torch.bfloat16, torch.float16)
                and (bias is None or (bias.dtype == tensor.dtype and bias.is_contiguous())))

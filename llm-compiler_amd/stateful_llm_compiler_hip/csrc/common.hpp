@@ -163,13 +163,31 @@ inline bool is_float_dtype(int dtype) {
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Decode-sized linear shared by slc_hip_linear and the fused decode ops
-// (defined with those kernels).
-// Prefill-sized linear + residual add (linear.hip); SLC_ERR_UNSUPPORTED when
-// its kernel does not take the shape.
+// Whether a 33 to 64-row linear of this many features runs on 64 x 64 ring tiles
+// rather than on the row kernel, which also splits K over its waves.  The tiles
+// need enough of them to fill the chip (33 | 48 | 64 rows, us, weights not in L2,
+// row kernel then tiles): N11008 K896 14.5|15.8|17.6 then 8.7|9.4|9.7, N11008
+// K4096 44|51|58 then 26|27|29, N4096 K4096 18.1|21.1|24.6 then 19.4|20.5|22.3,
+// but N896 K4096 14.1|16.6|20.4 then 18.3|19.2|20.8.  Narrow short ones come out
+// even alone (N896 K896 5.0|5.6|6.4 then 5.4|5.4|5.6) and lose inside a layer,
+// where each launch brings another kernel's code in (six layers of width 896 at
+// 48 rows: all on the row kernel 397 us, only the wide ones on tiles 386, all
+// with K <= 3072 on tiles 400).  One rule for the single and the fused forms, so
+// their bits agree.
+inline bool rows_on_tiles(int64_t features) { return features >= 4096; }
+
+// Linears of more than 32 rows with a residual add, SwiGLU or up to three
+// weights on the tile kernel (linear.hip); SLC_ERR_UNSUPPORTED (nothing
+// launched) when it does not take the shape.
 int gemm_residual(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                   const void* w, const void* bias, const void* residual, int64_t r_rs, void* y,
                   int64_t y_rs, int dtype, hipStream_t stream);
+int gemm_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
+                const void* w_gate, const void* w_up, void* y, int64_t y_rs, int dtype,
+                hipStream_t stream);
+int gemm_group(const void* x, int64_t x_rs, int64_t rows, int64_t K, int count,
+               const void* const* w, const void* const* bias, void* const* y,
+               const int64_t* n, const int64_t* y_rs, int dtype, hipStream_t stream);
 // fp32 linear on the fp32 matrix cores (linear_f32.hip); SLC_ERR_UNSUPPORTED
 // (nothing launched) for shapes its kernels do not take.
 int linear_f32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
@@ -195,6 +213,8 @@ int decode_attention_f32(const float* query, const float* kb, const float* vb, c
                          int64_t num_counters, int64_t batch, int64_t q_heads, int64_t kv_heads,
                          int64_t head_dim, int64_t capacity, int64_t mask_len,
                          const int64_t* strides, float scale, hipStream_t stream);
+// Decode-sized linear shared by slc_hip_linear and the fused decode ops
+// (defined with those kernels).
 bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                           int dtype);
 int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,

@@ -16,7 +16,8 @@
 //  * rope_kv_store       rope -> kv_store of the rotated keys and the values;
 //                        the rotated queries are written out.
 //
-// slc_hip_linear runs its decode-sized (<= 64 rows) cases on this same kernel
+// slc_hip_linear runs its decode-sized cases (up to 32 rows, and 33 to 64 where
+// rows_on_tiles says no) on this same kernel
 // (rows_linear), so a fused op and the ops it replaces share the K split over
 // the waves, the MFMA order and the partial-sum order, hence the same bits.
 // Semantics: src/stateful_llm_compiler/execution.py:674-692 (rms_norm),
@@ -847,6 +848,7 @@ extern "C" int slc_hip_linear_residual(const void* x, int64_t x_rs, int64_t rows
   const char* what = "slc_hip_linear_residual";
   if (rows > kMaxRows) {
     // Prefill-sized: the tile kernel with the residual in its store epilogue.
+    if (rows <= 64) return SLC_ERR_UNSUPPORTED;
     SLC_REQUIRE(x && weight && residual && y && in_features >= 1 && out_features >= 1,
                 "%s: bad operands", what);
     return slc_host::gemm_residual(x, x_rs, rows, in_features, out_features, weight, bias,
@@ -875,7 +877,8 @@ extern "C" int slc_hip_linear_residual(const void* x, int64_t x_rs, int64_t rows
 
 // ---- 33 to 64 rows ----------------------------------------------------------
 // The fused forms without their norm (it ran before): up to three linears of
-// one input, the SwiGLU pair, the linear with its residual add.
+// one input, the SwiGLU pair, the linear with its residual add.  Each weight
+// runs where slc_hip_linear runs it: on the 64 x 64 tiles or on the row kernel.
 
 namespace {
 
@@ -911,18 +914,39 @@ extern "C" int slc_hip_rows_linear_group(const void* input, int64_t in_stride_ro
   void* ys[3] = {y0, y1, y2};
   const int64_t ns[3] = {n0, n1, n2};
   const int64_t rss[3] = {y0_rs, y1_rs, y2_rs};
+  hipStream_t s = static_cast<hipStream_t>(stream);
   FusedArgs a = plain_rows(input, in_stride_row, rows, in_features);
+  // Weights of both kinds (grouped-query K and V of a wide model beside its Q)
+  // make one launch of each; the tiles go first and decline before any launch.
+  const void* tw[3] = {};
+  const void* tb[3] = {};
+  void* ty[3] = {};
+  int64_t tn[3] = {}, trs[3] = {};
+  int tiled = 0, rowed = 0;
   for (int i = 0; i < count; ++i) {
     if (!plain_rows_ok(input, in_stride_row, rows, in_features, ns[i], ws[i], ys[i], rss[i], dtype))
       return SLC_ERR_UNSUPPORTED;
-    a.w[i] = ws[i];
-    a.bias[i] = bs[i];
-    a.y[i] = ys[i];
-    a.n[i] = static_cast<int>(ns[i]);
-    a.y_rs[i] = rss[i];
+    if (slc_host::rows_on_tiles(ns[i])) {
+      tw[tiled] = ws[i];
+      tb[tiled] = bs[i];
+      ty[tiled] = ys[i];
+      tn[tiled] = ns[i];
+      trs[tiled++] = rss[i];
+    } else {
+      a.w[rowed] = ws[i];
+      a.bias[rowed] = bs[i];
+      a.y[rowed] = ys[i];
+      a.n[rowed] = static_cast<int>(ns[i]);
+      a.y_rs[rowed++] = rss[i];
+    }
   }
-  assign_blocks(a, count);
-  return dispatch_rows<kStore>(a, dtype, static_cast<hipStream_t>(stream));
+  if (tiled > 0) {
+    const int rc = slc_host::gemm_group(input, in_stride_row, rows, in_features, tiled, tw, tb, ty,
+                                        tn, trs, dtype, s);
+    if (rc != SLC_OK || rowed == 0) return rc;
+  }
+  assign_blocks(a, rowed);
+  return dispatch_rows<kStore>(a, dtype, s);
 }
 
 extern "C" int slc_hip_rows_linear_swiglu(const void* input, int64_t in_stride_row, int64_t rows,
@@ -934,6 +958,9 @@ extern "C" int slc_hip_rows_linear_swiglu(const void* input, int64_t in_stride_r
     if (!plain_rows_ok(input, in_stride_row, rows, in_features, features, w, output, out_stride_row,
                        dtype))
       return SLC_ERR_UNSUPPORTED;
+  if (slc_host::rows_on_tiles(features))
+    return slc_host::gemm_swiglu(input, in_stride_row, rows, in_features, features, w_gate, w_up,
+                                 output, out_stride_row, dtype, static_cast<hipStream_t>(stream));
   FusedArgs a = plain_rows(input, in_stride_row, rows, in_features);
   a.w[0] = w_gate;
   a.w[1] = w_up;
@@ -956,6 +983,10 @@ extern "C" int slc_hip_rows_linear_residual(const void* input, int64_t in_stride
       !plain_rows_ok(input, in_stride_row, rows, in_features, out_features, weight, output,
                      out_stride_row, dtype))
     return SLC_ERR_UNSUPPORTED;
+  if (slc_host::rows_on_tiles(out_features))
+    return slc_host::gemm_residual(input, in_stride_row, rows, in_features, out_features, weight,
+                                   bias, residual, residual_stride_row, output, out_stride_row,
+                                   dtype, static_cast<hipStream_t>(stream));
   FusedArgs a = plain_rows(input, in_stride_row, rows, in_features);
   a.w[0] = weight;
   a.bias[0] = bias;

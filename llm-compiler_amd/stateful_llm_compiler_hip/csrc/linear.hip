@@ -1185,8 +1185,13 @@ template <typename T>
 int dispatch_mfma(const void* x, const void* w, const void* bias, void* y, int M,
                   int N, int K, int64_t x_rs, int64_t y_rs, hipStream_t s, int tile = SLC_TILE_AUTO) {
   // Up to 64 rows: the decode-step linear kernel the fused ops share (a
-  // vocabulary-wide output past 16 rows: the tiles below).
+  // vocabulary-wide output past 16 rows: the tiles below), except 33 to 64 rows
+  // of a wide weight, which 64 x 64 ring tiles stream faster (rows_on_tiles).
   const int dtype = sizeof(T) == 2 && std::is_same<T, slc::bf16_t>::value ? SLC_BF16 : SLC_F16;
+  if (M > 32 && M <= 64 && N < kWideOutputs && slc_host::rows_on_tiles(N)) {
+    const int rc = launch_ring_tile<T>(SLC_TILE_R64X64, x, w, bias, y, M, N, K, x_rs, y_rs, s);
+    if (rc != kNoResidualPath) return rc;
+  }
   if (M <= 64 && slc_host::rows_linear_eligible(x, x_rs, M, K, N, dtype))
     return slc_host::rows_linear(x, x_rs, M, K, N, w, bias, y, y_rs, dtype, s);
   if (M <= 16) return launch_skinny<T, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
@@ -1251,14 +1256,14 @@ int gemm_residual(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t 
                   int64_t y_rs, int dtype, hipStream_t stream) {
   const uint64_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
                         reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(y);
-  const bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 64 && (bits & 15) == 0 &&
+  const bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 32 && (bits & 15) == 0 &&
                   K % kBK == 0 && N % 8 == 0 && x_rs % 8 == 0 && y_rs % 8 == 0 &&
                   r_rs % 8 == 0 && N * K * 2 < (int64_t{1} << 31) &&
                   128 * x_rs * 2 < (int64_t{1} << 31) && 128 * y_rs * 2 < (int64_t{1} << 31) &&
                   128 * r_rs * 2 < (int64_t{1} << 31) && rows < (int64_t{1} << 31);
-  if (!ok) return SLC_ERR_UNSUPPORTED;
+  if (!ok || (rows <= 64 && N >= kWideOutputs)) return SLC_ERR_UNSUPPORTED;
   const int M = static_cast<int>(rows), n = static_cast<int>(N), k = static_cast<int>(K);
-  const int tile = auto_ring_tile(M, (n + 127) / 128);
+  const int tile = rows <= 64 ? SLC_TILE_R64X64 : auto_ring_tile(M, (n + 127) / 128);
   int rc = dtype == SLC_BF16
                ? launch_ring_tile<slc::bf16_t>(tile, x, w, bias, y, M, n, k, x_rs, y_rs, stream,
                                                residual, r_rs)
@@ -1282,9 +1287,10 @@ int gemm_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                 hipStream_t stream) {
   const uint64_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w_gate) |
                         reinterpret_cast<uintptr_t>(w_up) | reinterpret_cast<uintptr_t>(y);
-  const bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 64 && (bits & 15) == 0 &&
+  const bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 32 && (bits & 15) == 0 &&
                   K % kBK == 0 && N % 8 == 0 && x_rs % 8 == 0 && y_rs % 8 == 0 &&
-                  N * K * 2 < (int64_t{1} << 31) && 128 * x_rs * 2 < (int64_t{1} << 31) &&
+                  (rows > 64 || N < kWideOutputs) && N * K * 2 < (int64_t{1} << 31) &&
+                  128 * x_rs * 2 < (int64_t{1} << 31) &&
                   128 * y_rs * 2 < (int64_t{1} << 31) && rows < (int64_t{1} << 31);
   if (!ok) return SLC_ERR_UNSUPPORTED;
   const int M = static_cast<int>(rows), n = static_cast<int>(N), k = static_cast<int>(K);
@@ -1301,6 +1307,24 @@ int gemm_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                                                          (n + 63) / 64, stream, w_up);
     if (rc != kNoResidualPath) return rc;
   }
+  // Small grids: 64 x 64 tiles of 32 gate and 32 up features, two k-tiles per
+  // stage where K allows (M48 N2x4864 K896 8.8 us, the 128 x 128 tile 11.8, the
+  // row kernel 10.8; weights not in L2).
+#define SLC_DUAL64(TT, PW, S, KT)                                                                 \
+  hipLaunchKernelGGL((linear_ring_kernel<TT, 64, 64, 2, 2, PW, S, 8, true, false, KT>),           \
+                     dim3((n + 31) / 32, (M + 63) / 64), dim3((4 + PW) * 64), 0, stream,          \
+                     static_cast<const TT*>(x), static_cast<const TT*>(w_gate),                   \
+                     static_cast<const TT*>(nullptr), static_cast<TT*>(y), M, n, k, x_rs, y_rs,   \
+                     static_cast<const TT*>(nullptr), int64_t{0}, static_cast<const TT*>(w_up))
+  if (rows <= 64 || auto_ring_tile(M, (n + 63) / 64) == SLC_TILE_R64X64) {
+    if (dtype == SLC_BF16) {
+      if (k % (2 * kBK) == 0) SLC_DUAL64(slc::bf16_t, 2, 4, 2); else SLC_DUAL64(slc::bf16_t, 1, 5, 1);
+    } else {
+      if (k % (2 * kBK) == 0) SLC_DUAL64(slc::f16_t, 2, 4, 2); else SLC_DUAL64(slc::f16_t, 1, 5, 1);
+    }
+    return check_launch("slc_hip_linear_swiglu");
+  }
+#undef SLC_DUAL64
 #define SLC_DUAL(TT, BM, CWM, PW, S, GM)                                                          \
   hipLaunchKernelGGL((linear_ring_kernel<TT, BM, 128, CWM, 2 * 4 / CWM, PW, S, GM, true>),         \
                      dim3((n + 63) / 64, (M + BM - 1) / BM), dim3((8 + PW) * 64), 0, stream,      \
@@ -1322,14 +1346,15 @@ int gemm_swiglu(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
 int gemm_group(const void* x, int64_t x_rs, int64_t rows, int64_t K, int count,
                const void* const* w, const void* const* bias, void* const* y,
                const int64_t* n, const int64_t* y_rs, int dtype, hipStream_t stream) {
-  bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 64 && count >= 1 && count <= 3 &&
+  bool ok = (dtype == SLC_BF16 || dtype == SLC_F16) && rows > 32 && count >= 1 && count <= 3 &&
             K % kBK == 0 && x_rs % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
             128 * x_rs * 2 < (int64_t{1} << 31) && rows < (int64_t{1} << 31);
   LinearGroup g{};
-  int tiles = 0;
+  int tiles = 0, tiles64 = 0, end64[3] = {};
   for (int j = 0; j < 3; ++j) {
     if (j < count) {
-      ok = ok && w[j] != nullptr && y[j] != nullptr && n[j] >= 1 && n[j] % 8 == 0 &&
+      ok = ok && (rows > 64 || n[j] < kWideOutputs) && w[j] != nullptr && y[j] != nullptr &&
+           n[j] >= 1 && n[j] % 8 == 0 &&
            y_rs[j] % 8 == 0 && y_rs[j] >= n[j] && n[j] * K * 2 < (int64_t{1} << 31) &&
            128 * y_rs[j] * 2 < (int64_t{1} << 31) &&
            ((reinterpret_cast<uintptr_t>(w[j]) | reinterpret_cast<uintptr_t>(y[j])) & 15) == 0;
@@ -1340,11 +1365,32 @@ int gemm_group(const void* x, int64_t x_rs, int64_t rows, int64_t K, int count,
       g.n[j] = static_cast<int>(n[j]);
       g.y_rs[j] = y_rs[j];
       tiles += static_cast<int>((n[j] + 127) / 128);
+      tiles64 += static_cast<int>((n[j] + 63) / 64);
     }
     g.tile_end[j] = tiles;
+    end64[j] = tiles64;
   }
   if (!ok) return SLC_ERR_UNSUPPORTED;
   const int M = static_cast<int>(rows), k = static_cast<int>(K);
+  // Small grids: 64 x 64 tiles (M72 K896 896 + 128 + 128 8.1 -> 5.7 us, M128
+  // 8.5 -> 5.9).
+#define SLC_GROUP64(TT, PW, S, KT)                                                               \
+  hipLaunchKernelGGL((linear_ring_kernel<TT, 64, 64, 2, 2, PW, S, 8, false, true, KT>),          \
+                     dim3(static_cast<unsigned>(tiles64), (M + 63) / 64), dim3((4 + PW) * 64), 0, \
+                     stream, static_cast<const TT*>(x), static_cast<const TT*>(nullptr),         \
+                     static_cast<const TT*>(nullptr), static_cast<TT*>(nullptr), M, 0, k, x_rs,  \
+                     int64_t{0}, static_cast<const TT*>(nullptr), int64_t{0},                    \
+                     static_cast<const TT*>(nullptr), g)
+  if (rows <= 64 || auto_ring_tile(M, tiles) == SLC_TILE_R64X64) {
+    for (int j = 0; j < 3; ++j) g.tile_end[j] = end64[j];
+    if (dtype == SLC_BF16) {
+      if (k % (2 * kBK) == 0) SLC_GROUP64(slc::bf16_t, 2, 4, 2); else SLC_GROUP64(slc::bf16_t, 1, 5, 1);
+    } else {
+      if (k % (2 * kBK) == 0) SLC_GROUP64(slc::f16_t, 2, 4, 2); else SLC_GROUP64(slc::f16_t, 1, 5, 1);
+    }
+    return check_launch("slc_hip_linear_group");
+  }
+#undef SLC_GROUP64
   bool big = auto_ring_tile(M, tiles) == SLC_TILE_R256X128 && 256 * x_rs * 2 < (int64_t{1} << 31);
   for (int j = 0; j < count; ++j) big = big && 256 * y_rs[j] * 2 < (int64_t{1} << 31);
 #define SLC_GROUP(TT, BM, CWM, PW, S, GM)                                                        \
@@ -1375,6 +1421,7 @@ extern "C" int slc_hip_linear_group(const void* input, int64_t in_stride_row, in
               "slc_hip_linear_group: bad sizes");
   if (rows == 0) return SLC_OK;
   SLC_REQUIRE(input != nullptr, "slc_hip_linear_group: null input");
+  if (rows <= 64) return SLC_ERR_UNSUPPORTED;
   const void* ws[3] = {w0, w1, w2};
   const void* bs[3] = {b0, b1, b2};
   void* ys[3] = {y0, y1, y2};
@@ -1392,6 +1439,7 @@ extern "C" int slc_hip_linear_swiglu(const void* input, int64_t in_stride_row, i
               "slc_hip_linear_swiglu: bad sizes");
   if (rows == 0) return SLC_OK;
   SLC_REQUIRE(input && w_gate && w_up && output, "slc_hip_linear_swiglu: null pointer");
+  if (rows <= 64) return SLC_ERR_UNSUPPORTED;
   return slc_host::gemm_swiglu(input, in_stride_row, rows, in_features, features, w_gate, w_up,
                                output, out_stride_row, dtype, static_cast<hipStream_t>(stream));
 }

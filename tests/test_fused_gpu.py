@@ -136,6 +136,41 @@ def test_plain_fused_ops_past_the_norm_rows(gpu, rows, hidden, features, dtype):
     assert ((single[1].double().cpu() - exact).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [33, 64, 65, 130])
+@pytest.mark.parametrize("hidden,ns", [(192, (4096, 4088, 8)), (128, (4104, 4096)), (72, (4096, 200)),
+                                       (64, (72, 136, 64))])
+def test_small_tiles_of_the_fused_projections(gpu, rows, hidden, ns, dtype):
+    """The 64 x 64 tiles of the grouped and SwiGLU forms, at the line to the
+    row kernel (4096 features up to 64 rows), with odd and even k-tiles, tile
+    remainders and a width that they decline: bit for bit the single linears,
+    which are within the bound of float64."""
+    announce(f"small tiles rows={rows} hidden={hidden} ns={ns} {dtype}")
+    g = generator(rows + hidden + len(ns))
+    x = _t(g, rows, 1, hidden, dtype=dtype, device=gpu)
+    ws = [_t(g, n, hidden, dtype=dtype, scale=0.05, device=gpu) for n in ns]
+    bs = [_t(g, n, dtype=dtype, scale=0.1, device=gpu) for n in ns]
+    single = [hip_linear(x, w, b) for w, b in zip(ws, bs)]
+    for got, want in zip(hip_norm_linear_group(x, None, ws, bs, epsilon=1e-6), single):
+        assert_bitwise_equal(got, want)
+    r = _t(g, rows, 1, ns[0], dtype=dtype, device=gpu)
+    assert_bitwise_equal(hip_linear_residual(x, ws[0], bs[0], r), hip_add(r, single[0]))
+    nw = _t(g, hidden, dtype=dtype, scale=0.5, device=gpu) + 1
+    xn = hip_rms_norm(x, nw, epsilon=1e-6, round_before_weight=True)
+    up = _t(g, ns[0], hidden, dtype=dtype, scale=0.05, device=gpu)
+    assert_bitwise_equal(hip_norm_linear_swiglu(x, nw, ws[0], up, epsilon=1e-6),
+                         hip_swiglu(hip_linear(xn, ws[0]), hip_linear(xn, up)))
+    unit = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    for w, b, y in zip(ws, bs, single):
+        x64, w64, b64 = x.double().cpu(), w.double().cpu(), b.double().cpu()
+        exact = x64 @ w64.T
+        # Two roundings to the type where the bias is added after the first,
+        # any order of an fp32 sum, and fp16's subnormal spacing.
+        bound = (2 * unit * (exact.abs() + b64.abs()) + (hidden + 2) * 2.0**-24 * (x64.abs() @ w64.abs().T)
+                 + 2.0**-23)
+        assert ((y.double().cpu() - exact - b64).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("tokens", [1, 5])
 def test_rope_kv_store_matches_rope_then_store(gpu, tokens):
     announce(f"rope_kv_store tokens={tokens}")
