@@ -3,8 +3,9 @@
 Each wrapper computes exactly what a short sequence of the single ops
 computes -- the fused kernels share those kernels' arithmetic, so the results
 are bit-identical -- in one launch when the input is decode-sized (at most 32
-rows of bf16/fp16), and by running that sequence of single-op kernels
-otherwise.  Both paths are HIP kernels; nothing runs on the host.
+rows of bf16/fp16), after a norm launch of its own from 33 rows on, and by
+running that sequence of single-op kernels where no fused kernel takes the
+shape.  Both paths are HIP kernels; nothing runs on the host.
 
 The sequences replaced (reference semantics):
   norm_linear_group   rms_norm (round_before_weight) -> 1..3 linears

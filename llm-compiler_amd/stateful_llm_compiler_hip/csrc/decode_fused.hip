@@ -397,9 +397,9 @@ int launch_rows(FusedArgs& a, hipStream_t stream) {
     // 33 .. 64 rows: three or four blocks of 16 input rows share every weight
     // read; the input rows come from the cache, each wave its own k-slice
     // (which bounds long K: each further block of 16 rows costs 4 us at K =
-    // 4864, whether 56 or 224 workgroups share the features).  M48 N4864 K896
-    // 10.0 -> 7.4 us, M48 N896 K4864 19 -> 17, and the MLP's five launches
-    // become three: 54 -> 29 us at 48 rows.
+    // 4864, whether 56 or 224 workgroups share the features).  M48 N896
+    // K4864 19 -> 17 us; weights of 4096 features or more go to the tiles
+    // (rows_on_tiles).
     if (a.rows > 32) {
       constexpr int W = EPI == kSwiglu ? 1 : 2;  // k-steps in flight, within the registers
       if (tiles == 2)

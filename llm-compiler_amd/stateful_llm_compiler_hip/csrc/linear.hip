@@ -14,9 +14,10 @@
 //    chunks so the 16-row MFMA operand reads (ds_read_b128) are free of bank
 //    conflicts.  Two LDS buffers: tile k+1 is fetched into registers while
 //    tile k is multiplied.
-//  * Decode-sized M (<= 64) takes a dedicated weight-streaming kernel (split-K
-//    across the waves of a workgroup, see linear_skinny_kernel); prefill-sized
-//    M uses 128 x 128 tiles (MFMA-bound).
+//  * Decode-sized M (<= 64) streams the weight with K split across the waves
+//    of a workgroup: the fused ops' row kernel (decode_fused.hip) or, where its
+//    alignment does not hold, linear_skinny_kernel.  Wide weights past 32 rows
+//    and prefill-sized M use tiles fed through an LDS ring (MFMA-bound).
 // fp32 runs on the fp32 matrix cores (linear_f32.hip); shapes neither vector
 // path can take use a classic LDS-tiled FMA kernel.
 #include <type_traits>
