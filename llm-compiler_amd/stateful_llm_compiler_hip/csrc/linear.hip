@@ -1090,10 +1090,12 @@ int launch_ring(const void* x, const void* w, const void* bias, void* y, int M, 
 // The persistent 256 x 128 form (linear_stream_kernel): one workgroup per CU
 // (a multiple of 8, so each one's tiles stay on its XCD), or one per tile
 // when there are fewer tiles.  kNoResidualPath where the shape does not fit.
-// The library launches it for plain linears and gate/up + SwiGLU from two rounds
-// of tiles on: its stores drain under the next tile's MFMAs, where the ring
-// kernel's workgroups end with them (M4096 N4864 K896 43.9 -> 40.1 us, M8192
-// 73.9 -> 66.3, M32768 341 -> 308, vocabulary head of 4096 rows 1270 -> 1202).
+// The library launches it for every plain linear of 256 x 128 tiles: its stores
+// drain under the next tile's MFMAs, where the ring kernel's workgroups end with
+// them (M4096 N4864 K896 43.9 -> 40.1 us, M8192 73.9 -> 66.3, M32768 341 -> 308,
+// vocabulary head of 4096 rows 1270 -> 1202), and with one tile per workgroup it
+// is ahead by its wider stores from registers (M8192 N896 K4864 63.9 -> 62.2, K896
+// 17.9 -> 17.1; M9362 K896 29.4 -> 26.4).  Gate/up + SwiGLU: see stream_grid.
 template <typename T, bool DUAL>
 int launch_stream(const void* x, const void* w, const void* bias, void* y, int M, int N, int K,
                   int64_t x_rs, int64_t y_rs, int n_tiles, hipStream_t stream,
@@ -1113,8 +1115,8 @@ int launch_stream(const void* x, const void* w, const void* bias, void* y, int M
   return slc_host::check_launch("slc_hip_linear(stream)");
 }
 
-// Whether the persistent form takes a 256 x 128 grid of `tiles` output tiles:
-// from SLC_STREAM_MIN_ROUNDS rounds of one workgroup per CU.
+// Whether the persistent form takes a 256 x 128 gate/up grid of `tiles` output
+// tiles: from SLC_STREAM_MIN_ROUNDS rounds of one workgroup per CU.
 inline bool stream_grid(int64_t tiles) {
   return SLC_STREAM_MIN_ROUNDS > 0 &&
          tiles >= int64_t{SLC_STREAM_MIN_ROUNDS} * slc_host::device_cu_count();
@@ -1206,9 +1208,7 @@ int dispatch_mfma(const void* x, const void* w, const void* bias, void* y, int M
   // the variants differ in speed only, never in a bit of the result.
   if (tile == SLC_TILE_AUTO) {
     tile = wide_on_register_tiles(M, N) ? SLC_TILE_128X128 : auto_ring_tile(M, (N + 127) / 128);
-    // Two rounds of 256 x 128 tiles or more: the persistent form.
-    if (tile == SLC_TILE_R256X128 && stream_grid(int64_t{(M + 255) / 256} * ((N + 127) / 128)))
-      tile = SLC_TILE_S256X128;
+    if (tile == SLC_TILE_R256X128) tile = SLC_TILE_S256X128;
   }
   switch (tile) {
     case SLC_TILE_128X64:
