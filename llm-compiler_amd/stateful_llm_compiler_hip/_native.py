@@ -200,8 +200,9 @@ def current_stream(device: torch.device) -> int:
     a small linear call's 8.6 us on the host, twice that in the calls that also
     look up the stream's workspace (decode attention 15.2 -> 11.7 us)."""
 
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    return torch._C._cuda_getCurrentRawStream(index)
+    if device.index is None:  # a CPU tensor's device, which torch refuses
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def check(status: int, what: str) -> None:

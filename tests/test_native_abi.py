@@ -166,3 +166,13 @@ def test_stream_workspaces_are_bounded(monkeypatch):
         _native.stream_workspace(torch.device("cuda", 0))
     assert len(_native._stream_workspaces) == _native.MAX_STREAM_WORKSPACES
     assert first not in _native._stream_workspaces.values()
+
+
+def test_current_stream_refuses_a_device_without_index(monkeypatch):
+    import torch
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 7)
+    with pytest.raises((RuntimeError, ValueError)):
+        _native.current_stream(torch.device("cpu"))
+    assert _native.current_stream(torch.device("cuda", 0)) == 7
