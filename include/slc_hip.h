@@ -466,7 +466,9 @@ SLC_API int slc_hip_argmax(const void* logits, int64_t* output, int dtype, int64
  * bit-identically what that sequence of this library's kernels produces).
  * rows <= 32 (decode-sized), dtype bf16 or fp16, 16-byte aligned rows; larger
  * or other inputs are rejected with SLC_ERR_INVALID_ARGUMENT and the caller
- * runs the unfused sequence.
+ * runs the unfused sequence.  Without a norm the input rows, and in any form 16
+ * rows of a weight, have to span less than 2^31 bytes: SLC_ERR_UNSUPPORTED
+ * (nothing launched) otherwise.
  *
  *   norm_linear_group : y_j = linear(rms_norm(x, norm_weight), w_j, b_j) for
  *                       count = 1..3 matrices [n_j, hidden] (Q/K/V); no norm
@@ -532,7 +534,8 @@ SLC_API int slc_hip_rope_kv_store(
  * ops as for the entry points above).  bf16 or fp16, 16-byte aligned inputs
  * and weights, in_features and in_stride_row multiples of 8; features up to
  * 16368; from 4096 features on also 16-byte aligned outputs, in_features a
- * multiple of 64, features and all strides multiples of 8.
+ * multiple of 64, features and all strides multiples of 8.  A weight and 128
+ * input rows (128 * in_stride_row elements) each span less than 2^31 bytes.
  * SLC_ERR_UNSUPPORTED (nothing launched) otherwise.
  */
 SLC_API int slc_hip_rows_linear_group(const void* input, int64_t in_stride_row, int64_t rows,

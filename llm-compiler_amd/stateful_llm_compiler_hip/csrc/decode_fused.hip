@@ -618,7 +618,17 @@ int dispatch_rows(FusedArgs& a, int dtype, hipStream_t stream) {
 #undef SLC_ROWS
 }
 
-// Shared argument checks: decode-sized rows, 16-byte aligned contiguous rows.
+// The row kernel reads its input rows (without a norm, which loads them by
+// 64-bit addresses) and 16 weight rows at 32-bit byte offsets inside ranges of
+// less than 2^31 bytes.  Past that, rows would read as zero or from elsewhere.
+bool row_offsets_fit(int64_t x_rs, int64_t rows, int64_t K, bool norm) {
+  constexpr int64_t kElements = int64_t{1} << 30;  // 16-bit elements of 2^31 bytes
+  return K < kElements / 16 &&
+         (norm || rows <= 1 || x_rs <= (kElements - 1 - K) / (rows - 1));
+}
+
+// Shared argument checks: decode-sized rows, 16-byte aligned contiguous rows,
+// and (SLC_ERR_UNSUPPORTED) rows within the kernel's 32-bit offsets.
 int check_rows(const char* what, const void* x, int64_t x_rs, int64_t rows, int64_t hidden,
                int dtype, bool norm) {
   SLC_REQUIRE(dtype == SLC_BF16 || dtype == SLC_F16, "%s: dtype must be bf16 or fp16", what);
@@ -629,6 +639,7 @@ int check_rows(const char* what, const void* x, int64_t x_rs, int64_t rows, int6
   SLC_REQUIRE(x != nullptr && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && x_rs >= hidden &&
                   x_rs % 8 == 0,
               "%s: input rows must be 16-byte aligned", what);
+  if (!row_offsets_fit(x_rs, rows, hidden, norm)) return SLC_ERR_UNSUPPORTED;
   return SLC_OK;
 }
 
@@ -883,12 +894,14 @@ extern "C" int slc_hip_linear_residual(const void* x, int64_t x_rs, int64_t rows
 namespace {
 
 // Whether the row kernel takes these rows and this weight; nothing is
-// launched otherwise.
+// launched otherwise.  The last line: slc_hip_linear's own limits, so that a
+// fused form never takes rows whose single linear runs on another kernel.
 bool plain_rows_ok(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N, const void* w,
                    const void* y, int64_t y_rs, int dtype) {
   return rows > kMaxRows && x != nullptr && w != nullptr && y != nullptr && x_rs >= K && N >= 1 &&
          y_rs >= N && (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
-         slc_host::rows_linear_eligible(x, x_rs, rows, K, N, dtype);
+         slc_host::rows_linear_eligible(x, x_rs, rows, K, N, dtype) &&
+         K < (int64_t{1} << 30) && N * K < (int64_t{1} << 30) && x_rs < (int64_t{1} << 30) / 128;
 }
 FusedArgs plain_rows(const void* x, int64_t x_rs, int64_t rows, int64_t K) {
   FusedArgs a{};

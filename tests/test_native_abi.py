@@ -138,6 +138,33 @@ def test_row_kernel_entry_points_decline_other_rows():
         assert call(k=0) == -1
 
 
+def test_row_kernel_entry_points_decline_offsets_past_32_bits():
+    # The row kernel addresses its input rows and 16 weight rows with 32-bit
+    # byte offsets: a row stride or a width past them is declined before a
+    # launch (no pointer is dereferenced), never read from a wrong place.
+    lib = _native.library()
+    p, bf16 = 0x1000, 2
+
+    def rows_forms(rows, stride, k, n):
+        yield lib.slc_hip_rows_linear_group(p, stride, rows, k, 1, p, None, p, n, n, None, None, None, 0, 0,
+                                            None, None, None, 0, 0, bf16, None)
+        yield lib.slc_hip_rows_linear_swiglu(p, stride, rows, k, n, p, p, p, n, bf16, None)
+        yield lib.slc_hip_rows_linear_residual(p, stride, rows, k, n, p, None, p, n, p, n, bf16, None)
+
+    def decode_forms(rows, stride, k, n):
+        yield lib.slc_hip_norm_linear_group(p, stride, None, 0.0, rows, k, 1, p, None, p, n, n, None, None, None, 0,
+                                            0, None, None, None, 0, 0, bf16, None)
+        yield lib.slc_hip_linear_residual(p, stride, rows, k, n, p, None, p, n, p, n, bf16, None)
+
+    # 128 rows of 2^23 elements and a weight of 2^30 are 2^31 bytes.
+    for rows, stride, k, n in ((40, 2**25, 896, 128), (33, 2**23, 896, 128), (64, 2**40, 896, 128),
+                               (40, 2**24, 2**24, 64), (40, 2**20, 2**20, 1024), (40, 2**34, 2**34, 8)):
+        assert list(rows_forms(rows, stride, k, n)) == [-2, -2, -2], (rows, stride, k, n)
+    for rows, stride, k, n in ((32, 2**30 // 31 // 8 * 8 + 8, 896, 128), (2, 2**30, 896, 128), (17, 2**40, 896, 128),
+                               (1, 2**26, 2**26, 16), (1, 2**36, 2**36, 16)):
+        assert list(decode_forms(rows, stride, k, n)) == [-2, -2], (rows, stride, k, n)
+
+
 def test_paged_kv_store_rejects_a_grid_past_one_launch():
     # 2^43 16-byte units need 2^35 workgroups of 256, past a launch: rejected on
     # the host (the pointers are never dereferenced).
