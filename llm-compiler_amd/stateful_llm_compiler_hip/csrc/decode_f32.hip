@@ -65,7 +65,8 @@ __global__ __launch_bounds__(kThreads) void decode_attention_f32_kernel(
   end64 = end64 < 0 ? 0 : end64;
   end64 = end64 < mask_len ? end64 : mask_len;
   end64 = end64 < capacity ? end64 : capacity;
-  // One sequence's length: uniform, and below 2^30 (the host checks).
+  // One sequence's length: uniform, and below 2^30 as a chunk's end is (the
+  // host checks).
   const int seq_end = __builtin_amdgcn_readfirstlane(static_cast<int>(end64));
   const int first = chunk * chunk_tokens;
   const int end = min(seq_end, first + chunk_tokens);
@@ -245,7 +246,7 @@ int decode_attention_f32(const float* query, const float* kb, const float* vb, c
   const int64_t groups = q_heads / kv_heads;
   if (!decode_f32_eligible(head_dim, groups) || mask_len < 1 || (bits & 15) != 0 ||
       (strides & 3) != 0 || st[3] < head_dim || st[3] >= (int64_t{1} << 24) ||
-      std::min(mask_len, capacity) >= (int64_t{1} << 30))
+      mask_len >= (int64_t{1} << 30))
     return SLC_ERR_UNSUPPORTED;
   int64_t n = decode_f32_chunks(batch, q_heads, kv_heads, head_dim, mask_len);
   // Without room for the partials one workgroup takes a whole sequence.

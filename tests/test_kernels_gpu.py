@@ -419,6 +419,22 @@ def test_decode_fp32_matrix_cores(gpu, batch, q_heads, kv_heads, head_dim, capac
     assert_fp32_close(actual[~empty], expected[~empty])
 
 
+def test_decode_fp32_mask_past_32_bit_chunks(gpu):
+    # A mask far longer than the cache (one zero, expanded): a chunk of 2^31
+    # tokens has no 32-bit end, and these 520 sequences take one chunk each.
+    from stateful_llm_compiler_hip.backends import hip_decode_attention
+
+    announce("decode fp32 B=520 cap=8 mask of 2^31 entries")
+    g = generator(17)
+    q, k, v = (torch.randn(520, *shape, generator=g) for shape in ((2, 1, 64), (8, 1, 64), (8, 1, 64)))
+    lengths = torch.randint(1, 9, (520,), generator=g)
+    expected = ref.decode_attention(q, k, v, lengths, torch.zeros(520, 1, 1, 8), groups=2, scale=0.125)
+    mask = torch.zeros(1, 1, 1, 1, device=gpu).expand(520, 1, 1, 2**31)
+    actual = hip_decode_attention(q.to(gpu), k.to(gpu), v.to(gpu), lengths.to(gpu), mask, scale=0.125)
+    torch.cuda.synchronize()
+    assert_fp32_close(actual, expected)
+
+
 @pytest.mark.parametrize("waves", [None, 1, 4])
 @pytest.mark.parametrize("rows", [1, 8, 64, 512, 32768])
 def test_rms_norm_bf16_round_before_weight(gpu, rows, waves):
