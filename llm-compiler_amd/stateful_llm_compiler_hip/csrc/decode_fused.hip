@@ -764,7 +764,7 @@ int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
   a.y[0] = y;
   a.n[0] = static_cast<int>(N);
   a.y_rs[0] = y_rs;
-  if ((N + 15) / 16 >= kWideBlocks) {
+  if (rows <= 16 && (N + 15) / 16 >= kWideBlocks) {
     return dtype == SLC_BF16 ? launch_wide<slc::bf16_t>(a, stream)
                              : launch_wide<slc::f16_t>(a, stream);
   }

@@ -1138,15 +1138,45 @@ inline int auto_ring_tile(int64_t M, int64_t n_tiles128) {
   return n128 >= 300 ? SLC_TILE_R256X128 : SLC_TILE_R128X128;
 }
 
-// Vocabulary-wide outputs write as many bytes as they read, and three
-// register-staged 128 x 128 workgroups per CU overlap one's stores with the
-// others' loads: with up to 128 rows they stream the weights (M65 N151936
-// 51.9 us, the 256 x 128 ring 82.2, the skinny kernel 180 at M64), and they
-// win whenever 256-row tiles would leave half a tile empty (M300 128.5 against
-// 150.4; M1000 334.5 against 328.7).
+// Features from which linears of 17 to 64 rows leave the row kernels for tiles.
 constexpr int kWideOutputs = 16384;
-inline bool wide_on_register_tiles(int64_t M, int64_t N) {
-  return N >= kWideOutputs && ((M + 127) / 128) % 2 == 1;
+
+// Tile of a plain linear when the caller leaves it to the library.  `ring`: the
+// ring kernels take the shape (K in whole k-tiles, 16-byte stores).  Where
+// auto_ring_tile says 256 x 128, the persistent form (launch_stream), except in
+// these cases for the register-staged 128 x 128 tile, three workgroups of which
+// share a CU and overlap one's stores with the others' loads (us, weights not in
+// cache, register-staged | persistent):
+//  * up to 128 rows, where half of a 256-row tile or more is empty: 20 rows
+//    N151936 K896 57 | 61, 64 rows N49152 K3072 69 | 73, 128 rows N200064 K1536
+//    164 | 168.  Not where a third of their rounds would be empty and K is long:
+//    ring 128 x 128, one per CU (128 rows N128256 K4096 255 | 238, ring 232, K1536
+//    114 | 101, ring 104);
+//  * an odd number of 128-row tiles of a vocabulary-wide output, where half a
+//    256-row tile is empty: with K up to 256 (300 rows N49152 K128 13.7 | 16.2,
+//    640 rows N24576 K256 16.8 | 18.7), where the 256-row grid is just past one
+//    round (300 rows N18944 K896 22 | 26, K4096 77 | 93; but 640 rows, 1.7
+//    rounds, 119 | 106), and with three such tiles of a very wide output (300
+//    rows N151936 K896 129 | 134; N98304 83 | 78, 640 rows N151936 222 | 199).
+// Everywhere else the half tile costs less than the register-staged kernel's
+// slower k-tiles (1100 rows N151936 K896 395 | 362, 4224 rows N16384 K4096 603 |
+// 477).  Without the ring: register-staged tiles of 128 x 128, or of 32 x 64 with
+// up to 32 rows, and up to 64 while the wide grid leaves CUs idle (32 x 64 | 128
+// x 128: 20 rows N28673 K4096 64 | 74; 64 rows N28673 K4096 66 | 76, N50257 K896
+// 32 | 24).
+inline int auto_tile(int64_t M, int64_t N, int64_t K, bool ring) {
+  const int64_t cus = slc_host::device_cu_count(), n_tiles = (N + 127) / 128, m_tiles = (M + 127) / 128;
+  if (!ring) return M <= 32 || (M <= 64 && n_tiles <= cus) ? SLC_TILE_32X64 : SLC_TILE_128X128;
+  const int tile = auto_ring_tile(M, n_tiles);
+  if (tile != SLC_TILE_R256X128) return tile;
+  if (m_tiles == 1) {
+    const int64_t round = 3 * cus, slots = (n_tiles + round - 1) / round * round;
+    return K >= 1024 && n_tiles > round && 2 * slots > 3 * n_tiles ? SLC_TILE_R128X128 : SLC_TILE_128X128;
+  }
+  const int64_t grid = n_tiles * ((m_tiles + 1) / 2);
+  const bool staged = N >= kWideOutputs && m_tiles % 2 == 1 && grid > cus &&
+                      (K <= 256 || 4 * grid <= 5 * cus || (m_tiles == 3 && K < 1024 && grid > 8 * cus));
+  return staged ? SLC_TILE_128X128 : SLC_TILE_S256X128;
 }
 
 // One of the ring tiles; kNoResidualPath (nothing launched) where the shape
@@ -1199,17 +1229,17 @@ int dispatch_mfma(const void* x, const void* w, const void* bias, void* y, int M
     return slc_host::rows_linear(x, x_rs, M, K, N, w, bias, y, y_rs, dtype, s);
   if (M <= 16) return launch_skinny<T, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
   if (M <= 32 && N < kWideOutputs) return launch_skinny<T, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-  if (M <= 64) {
-    if (N >= kWideOutputs) return launch_mfma<T, 128, 128, 2, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-    return launch_skinny<T, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-  }
-  // Tile variants (a profile plan picks one): every tile accumulates each
-  // output's k range in the same order, 32 k at a time on one MFMA chain, so
-  // the variants differ in speed only, never in a bit of the result.
-  if (tile == SLC_TILE_AUTO) {
-    tile = wide_on_register_tiles(M, N) ? SLC_TILE_128X128 : auto_ring_tile(M, (N + 127) / 128);
-    if (tile == SLC_TILE_R256X128) tile = SLC_TILE_S256X128;
-  }
+  if (M <= 64 && N < kWideOutputs) return launch_skinny<T, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
+  const bool ring = K % kBK == 0 && N % 8 == 0 && y_rs % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+  // Up to 32 rows without the ring: the row kernel while about two workgroups
+  // of 32 features per CU take all of N (us, 20 rows, row kernel | 32 x 64
+  // tiles: N16384 K1000 12.6 | 16.1, N17001 K4096 53 | 54, N28673 K4096 73 | 64).
+  if (M <= 32 && !ring && N <= 17408) return slc_host::rows_linear(x, x_rs, M, K, N, w, bias, y, y_rs, dtype, s);
+  // Tile variants (a profile plan picks one past 64 rows): every tile
+  // accumulates each output's k range in the same order, 32 k at a time on one
+  // MFMA chain, so the variants differ in speed only, never in a bit of the
+  // result.
+  if (tile == SLC_TILE_AUTO || M <= 64) tile = auto_tile(M, N, K, ring);
   switch (tile) {
     case SLC_TILE_128X64:
       return launch_mfma<T, 128, 64, 2, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);

@@ -92,6 +92,29 @@ def test_linear_bf16_vocabulary_width(gpu, rows, k, n, strided):
     _check_linear_bf16(y, x, w, None, against_oracle=False)
 
 
+@pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 128, 129, 300])
+@pytest.mark.parametrize("n,k", [
+    (16369, 72), (16376, 128), (16384, 1000), (17408, 40), (17409, 64),  # row kernel, 64 x 64, 32 x 64
+    (32769, 40), (18944, 192),                                           # no ring past one round; 128 x 128
+    (38400, 64), (38400, 2048)])                                         # 256-wide grids: short K, long K
+def test_linear_bf16_wide_tiles(gpu, rows, n, k):
+    """Wide outputs past the decode rows: each side of every line that
+    chooses their kernel (rows, whole k-tiles and 16-byte stores, grid
+    rounds, K) against the fp64 product."""
+
+    from stateful_llm_compiler_hip.backends import hip_linear
+
+    announce(f"linear bf16 wide M={rows} N={n} K={k}")
+    g = torch.Generator(device=gpu).manual_seed(rows + n + k)
+    x = torch.randn(rows, k, generator=g, device=gpu, dtype=torch.bfloat16)
+    w = torch.randn(n, k, generator=g, device=gpu, dtype=torch.bfloat16) * 0.02
+    b = torch.randn(n, generator=g, device=gpu, dtype=torch.bfloat16) * 0.02
+    y = hip_linear(x, w, b)
+    exact, terms = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T
+    # One bf16 ulp and the worst fp32 accumulation error, as above.
+    assert ((y.double() - exact).abs() <= _bf16_ulp(exact) + k * 2.0**-24 * (terms + b.double().abs()) + 1e-6).all()
+
+
 def test_linear_bf16_large_m_and_3d(gpu):
     from stateful_llm_compiler_hip.backends import hip_linear
 
