@@ -213,6 +213,12 @@ int decode_attention_f32(const float* query, const float* kb, const float* vb, c
                          int64_t num_counters, int64_t batch, int64_t q_heads, int64_t kv_heads,
                          int64_t head_dim, int64_t capacity, int64_t mask_len,
                          const int64_t* strides, float scale, hipStream_t stream);
+// Features from which a linear is vocabulary-wide: 1024 blocks of 16 fill the
+// GPU without splitting K, so up to 16 rows run one wave per block
+// (decode_fused.hip), and more rows on tiles (linear.hip) rather than on the row
+// kernel (20 rows N16376 K896 12.5 us, 64 x 64 tiles 8.7).
+constexpr int64_t kWideOutputs = 16 * 1023 + 1;
+
 // Decode-sized linear shared by slc_hip_linear and the fused decode ops
 // (defined with those kernels).
 bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,

@@ -425,11 +425,10 @@ int launch_rows(FusedArgs& a, hipStream_t stream) {
   return go(fused_rows_kernel<T, 2, 8, U2, NV, EPI, 1>, 2);
 }
 
-// Wide projections (the vocabulary head): enough 16-feature blocks to fill
-// the GPU without splitting K, so each wave owns one block over the whole K
-// (no cross-wave reduction, nothing through LDS) and keeps U k-steps of
-// weights in flight.
-constexpr int kWideBlocks = 1024;
+// Wide projections (the vocabulary head, kWideOutputs features or more): enough
+// 16-feature blocks to fill the GPU without splitting K, so each wave owns one
+// block over the whole K (no cross-wave reduction, nothing through LDS) and keeps
+// U k-steps of weights in flight.
 // XL: the input rows are staged in LDS once per workgroup (row stride K + 8
 // elements, so the 16 rows of an operand read fall 4 banks apart) instead of
 // being re-read from the cache by every wave at every k-step.
@@ -749,8 +748,9 @@ __global__ __launch_bounds__(256) void rope_kv_store_kernel(
 
 namespace slc_host {
 
-// Decode-sized plain linear (rows <= 32) for slc_hip_linear: the same kernel
-// as the fused ops, so fused and unfused graphs agree bit for bit.
+// Decode-sized plain linear (up to 64 rows) for slc_hip_linear: the same kernel
+// as the fused ops, so fused and unfused graphs agree bit for bit; the wide
+// kernel for a vocabulary-wide output of up to 16 rows.
 int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
                 const void* w, const void* bias, void* y, int64_t y_rs, int dtype,
                 hipStream_t stream) {
@@ -764,7 +764,7 @@ int rows_linear(const void* x, int64_t x_rs, int64_t rows, int64_t K, int64_t N,
   a.y[0] = y;
   a.n[0] = static_cast<int>(N);
   a.y_rs[0] = y_rs;
-  if (rows <= 16 && (N + 15) / 16 >= kWideBlocks) {
+  if (rows <= 16 && N >= kWideOutputs) {
     return dtype == SLC_BF16 ? launch_wide<slc::bf16_t>(a, stream)
                              : launch_wide<slc::f16_t>(a, stream);
   }
@@ -776,7 +776,7 @@ bool rows_linear_eligible(const void* x, int64_t x_rs, int64_t rows, int64_t K, 
                           int dtype) {
   return (dtype == SLC_BF16 || dtype == SLC_F16) && rows >= 1 && rows <= kMaxPlainRows &&
          K % 8 == 0 && K >= 8 && x_rs % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
-         N <= (1 << 24) && (rows <= 16 || (N + 15) / 16 < kWideBlocks);
+         (rows <= 16 || N < kWideOutputs);
 }
 
 }  // namespace slc_host
@@ -818,7 +818,7 @@ extern "C" int slc_hip_norm_linear_group(
   // when that kernel cannot take the norm (rows past 16) nothing is launched
   // and the caller runs the norm and the linear: the equal-workgroup kernel
   // would sum K in another order.
-  if (count == 1 && (a.n[0] + 15) / 16 >= kWideBlocks && norm_weight != nullptr) {
+  if (count == 1 && a.n[0] >= slc_host::kWideOutputs && norm_weight != nullptr) {
     return dtype == SLC_BF16 ? launch_wide<slc::bf16_t>(a, static_cast<hipStream_t>(stream))
                              : launch_wide<slc::f16_t>(a, static_cast<hipStream_t>(stream));
   }

@@ -15,9 +15,9 @@
 //    conflicts.  Two LDS buffers: tile k+1 is fetched into registers while
 //    tile k is multiplied.
 //  * Decode-sized M (<= 64) streams the weight with K split across the waves
-//    of a workgroup: the fused ops' row kernel (decode_fused.hip) or, where its
-//    alignment does not hold, linear_skinny_kernel.  Wide weights past 32 rows
-//    and prefill-sized M use tiles fed through an LDS ring (MFMA-bound).
+//    of a workgroup: the fused ops' row kernel (decode_fused.hip).  Wide weights
+//    past 32 rows, vocabulary-wide ones past 16 and prefill-sized M use tiles
+//    fed through an LDS ring (MFMA-bound).
 // fp32 runs on the fp32 matrix cores (linear_f32.hip); shapes neither vector
 // path can take use a classic LDS-tiled FMA kernel.
 #include <type_traits>
@@ -31,7 +31,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
-typedef int i32x2_t __attribute__((ext_vector_type(2)));
 
 template <typename T>
 struct Mfma;
@@ -897,114 +896,6 @@ __global__ __launch_bounds__(12 * 64) void linear_stream_kernel(
   }
 }
 
-// Decode-sized M (<= 64): Y is a handful of rows, W streams from HBM once.
-// One workgroup owns 16 output features and all M rows; its KW waves split K
-// between them (partial sums meet in LDS at the end), so even a 896-wide
-// projection launches N/16 workgroups x KW waves.  Operands are loaded
-// straight into MFMA registers -- lane (row c, k-slice g) takes 16 bytes of
-// one W row per k-step -- U k-steps per batch, the next batch in flight while
-// the current one is multiplied.
-template <typename T, int MB, int KW, int U>
-__global__ __launch_bounds__(KW * 64) void linear_skinny_kernel(
-    const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ bias,
-    T* __restrict__ y, int M, int N, int K, int64_t x_rs, int64_t y_rs) {
-  using MF = Mfma<T>;
-  __shared__ float partial[KW][MB][64][4];
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int c = lane & 15;
-  const int g = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-
-  const int steps = (K + 31) / 32;               // 32-wide MFMA k-steps
-  const int per_wave = (steps + KW - 1) / KW;
-  const int s_begin = wave * per_wave;
-  const int s_end = min(s_begin + per_wave, steps);
-
-  const int w_rows = min(16, N - n0);
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(w + static_cast<int64_t>(n0) * K,
-                                              static_cast<int64_t>(w_rows) * K * 2);
-  const __amdgpu_buffer_rsrc_t rx =
-      make_rsrc(x, (static_cast<int64_t>(M) - 1) * x_rs * 2 + static_cast<int64_t>(K) * 2);
-  // Per-lane byte offsets of k-step 0; rows past N / M read zero.
-  const int w_off = c * K * 2 + g * 16;
-  int x_off[MB];
-#pragma unroll
-  for (int i = 0; i < MB; ++i) x_off[i] = static_cast<int>((i * 16 + c) * x_rs * 2) + g * 16;
-
-  f32x4_t acc[MB];
-#pragma unroll
-  for (int i = 0; i < MB; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  uint4 wa[U], xa[U][MB], wb[U], xb[U][MB];
-  auto fetch = [&](int s0, uint4 (&wr)[U], uint4 (&xr)[U][MB]) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = s0 + u;
-      const int k = s * 32 + g * 8;
-      // k past K (or past this wave's range) contributes zeros; within a row
-      // the buffer range check cannot see the end, so this lane test does.
-      const bool ok = s < s_end && k < K;
-      wr[u] = ok ? buffer_load16(rw, w_off + s * 64) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-        xr[u][i] = ok ? buffer_load16(rx, x_off[i] + s * 64) : make_uint4(0, 0, 0, 0);
-    }
-  };
-  auto multiply = [&](const uint4 (&wr)[U], const uint4 (&xr)[U][MB]) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const auto b = __builtin_bit_cast(typename MF::vec, wr[u]);
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-        acc[i] = MF::run(__builtin_bit_cast(typename MF::vec, xr[u][i]), b, acc[i]);
-    }
-  };
-
-  int s0 = s_begin;
-  fetch(s0, wa, xa);
-  while (s0 < s_end) {
-    fetch(s0 + U, wb, xb);
-    multiply(wa, xa);
-    s0 += U;
-    if (s0 >= s_end) break;
-    fetch(s0 + U, wa, xa);
-    multiply(wb, xb);
-    s0 += U;
-  }
-
-  // C layout: lane (col c = feature, rows 4g..4g+3 = batch rows of block i).
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) partial[wave][i][lane][r] = acc[i][r];
-  __syncthreads();
-  for (int idx = tid; idx < MB * 64 * 4; idx += KW * 64) {
-    const int i = idx / 256, l = (idx / 4) % 64, r = idx % 4;
-    float sum = 0.0f;
-#pragma unroll
-    for (int v = 0; v < KW; ++v) sum += partial[v][i][l][r];
-    const int n = n0 + (l & 15);
-    const int m = i * 16 + 4 * (l >> 4) + r;
-    if (n < N && m < M) {
-      if (bias != nullptr) sum += slc::to_f32(bias[n]);
-      y[m * y_rs + n] = slc::from_f32<T>(sum);
-    }
-  }
-}
-
-template <typename T, int MB>
-int launch_skinny(const void* x, const void* w, const void* bias, void* y, int M, int N,
-                  int K, int64_t x_rs, int64_t y_rs, hipStream_t stream) {
-  // k-steps per prefetch batch: as deep as the registers allow.
-  constexpr int KW = 8, U = MB == 1 ? 8 : (MB == 2 ? 4 : 2);
-  hipLaunchKernelGGL((linear_skinny_kernel<T, MB, KW, U>), dim3((N + 15) / 16), dim3(KW * 64), 0,
-                     stream, static_cast<const T*>(x), static_cast<const T*>(w),
-                     static_cast<const T*>(bias), static_cast<T*>(y), M, N, K, x_rs, y_rs);
-  return slc_host::check_launch("slc_hip_linear(skinny)");
-}
-
 // Classic 16 x 16 LDS-tiled FMA GEMM for unaligned shapes.
 template <typename T>
 __global__ __launch_bounds__(256) void linear_generic_kernel(
@@ -1138,9 +1029,6 @@ inline int auto_ring_tile(int64_t M, int64_t n_tiles128) {
   return n128 >= 300 ? SLC_TILE_R256X128 : SLC_TILE_R128X128;
 }
 
-// Features from which linears of 17 to 64 rows leave the row kernels for tiles.
-constexpr int kWideOutputs = 16384;
-
 // Tile of a plain linear when the caller leaves it to the library.  `ring`: the
 // ring kernels take the shape (K in whole k-tiles, 16-byte stores).  Where
 // auto_ring_tile says 256 x 128, the persistent form (launch_stream), except in
@@ -1174,7 +1062,7 @@ inline int auto_tile(int64_t M, int64_t N, int64_t K, bool ring) {
     return K >= 1024 && n_tiles > round && 2 * slots > 3 * n_tiles ? SLC_TILE_R128X128 : SLC_TILE_128X128;
   }
   const int64_t grid = n_tiles * ((m_tiles + 1) / 2);
-  const bool staged = N >= kWideOutputs && m_tiles % 2 == 1 && grid > cus &&
+  const bool staged = N >= slc_host::kWideOutputs && m_tiles % 2 == 1 && grid > cus &&
                       (K <= 256 || 4 * grid <= 5 * cus || (m_tiles == 3 && K < 1024 && grid > 8 * cus));
   return staged ? SLC_TILE_128X128 : SLC_TILE_S256X128;
 }
@@ -1217,19 +1105,16 @@ int launch_ring_tile(int tile, const void* x, const void* w, const void* bias, v
 template <typename T>
 int dispatch_mfma(const void* x, const void* w, const void* bias, void* y, int M,
                   int N, int K, int64_t x_rs, int64_t y_rs, hipStream_t s, int tile = SLC_TILE_AUTO) {
-  // Up to 64 rows: the decode-step linear kernel the fused ops share (a
-  // vocabulary-wide output past 16 rows: the tiles below), except 33 to 64 rows
-  // of a wide weight, which 64 x 64 ring tiles stream faster (rows_on_tiles).
+  // Up to 64 rows: the decode-step linear kernel the fused ops share, except a
+  // vocabulary-wide output past 16 rows (the tiles below) and 33 to 64 rows of
+  // a wide weight, which 64 x 64 ring tiles stream faster (rows_on_tiles).
   const int dtype = sizeof(T) == 2 && std::is_same<T, slc::bf16_t>::value ? SLC_BF16 : SLC_F16;
-  if (M > 32 && M <= 64 && N < kWideOutputs && slc_host::rows_on_tiles(N)) {
+  if (M > 32 && M <= 64 && N < slc_host::kWideOutputs && slc_host::rows_on_tiles(N)) {
     const int rc = launch_ring_tile<T>(SLC_TILE_R64X64, x, w, bias, y, M, N, K, x_rs, y_rs, s);
     if (rc != kNoResidualPath) return rc;
   }
   if (M <= 64 && slc_host::rows_linear_eligible(x, x_rs, M, K, N, dtype))
     return slc_host::rows_linear(x, x_rs, M, K, N, w, bias, y, y_rs, dtype, s);
-  if (M <= 16) return launch_skinny<T, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-  if (M <= 32 && N < kWideOutputs) return launch_skinny<T, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-  if (M <= 64 && N < kWideOutputs) return launch_skinny<T, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
   const bool ring = K % kBK == 0 && N % 8 == 0 && y_rs % 8 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
   // Up to 32 rows without the ring: the row kernel while about two workgroups
   // of 32 features per CU take all of N (us, 20 rows, row kernel | 32 x 64

@@ -65,9 +65,9 @@ def test_linear_bf16_qwen_shapes(gpu, rows, k, n, bias):
                                               (24, 896, 20000, False)])
 def test_linear_bf16_vocabulary_width(gpu, rows, k, n, strided):
     """The vocabulary-width decode kernel (one wave per 16 features over all
-    of K; input rows staged in LDS when they are 16-byte aligned, read from
-    the cache otherwise, as a strided view here; rows past 16 take two
-    row blocks) within one bf16 ulp of the fp64 product."""
+    of K, the input rows staged in LDS while they fit), the generic kernel for
+    a strided view with unaligned rows, and the tiles that rows past 16 take,
+    within one bf16 ulp of the fp64 product."""
     from stateful_llm_compiler_hip.backends import hip_linear
 
     announce(f"linear bf16 vocabulary width M={rows} K={k} N={n} strided={strided}")
