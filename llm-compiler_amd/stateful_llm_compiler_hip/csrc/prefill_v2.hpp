@@ -227,6 +227,9 @@ __global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attenti
   if (wave == G) {
     // ---- producer ---------------------------------------------------------
     constexpr int kOps = (2 * kV2TileBytes + kMaskTile) / 1024;  // DMA ops per tile
+    // Tiles whose mask is loaded element by element (stage_mask) issue fewer, so
+    // a wait that leaves later tiles in flight would release one too early.
+    static_assert(MK == 0 || kV2Stages == 2, "a masked tile's loads are not counted: wait for all");
     const char* kbase = reinterpret_cast<const char*>(key + b * k_sb + kvh * k_sh);
     const char* vbase = reinterpret_cast<const char*>(value + b * v_sb + kvh * v_sh);
     const char* mbase = MK == 0 ? nullptr

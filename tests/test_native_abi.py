@@ -69,6 +69,20 @@ def test_argument_checks_fail_without_touching_a_device():
     assert lib.slc_hip_argmax_workspace_size(8) == 8 * 64 * 12
 
 
+@pytest.mark.parametrize("stages,compiles", [(2, True), (3, False)])
+def test_masked_prefill_takes_two_ring_stages_only(stages, compiles):
+    # A deeper ring's wait counts loads that an element-loaded mask tile does
+    # not issue: such a build has to fail, not to read a tile too early.
+    from stateful_llm_compiler_hip import build
+
+    source = build.CSRC / "prefill_attention_short.hip"
+    command = [build._hipcc(), *build.HIPCC_FLAGS, "--cuda-host-only", "-fsyntax-only",
+               f"-DSLC_PREFILL_STAGES={stages}", str(source)]
+    result = subprocess.run(command, capture_output=True, text=True)
+    assert (result.returncode == 0) == compiles, result.stderr
+    assert compiles or "a masked tile's loads are not counted" in result.stderr
+
+
 def test_product_never_imports_the_oracle():
     package = ROOT / "llm-compiler_amd" / "stateful_llm_compiler_hip"
     for source in package.rglob("*.py"):
