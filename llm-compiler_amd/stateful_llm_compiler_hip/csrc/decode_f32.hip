@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kThreads) void decode_attention_f32_kernel(
     if (__any(mx > m_run + kRescaleThreshold)) {
       mx = slc::max_xor32(slc::max_xor16(mx));
       const float m_new = fmaxf(m_run, mx);
-      const float alpha = fast_exp2(m_run - (m_new == -INFINITY ? 0.0f : m_new));
+      const float alpha = weight_exp2<float>(m_run - (m_new == -INFINITY ? 0.0f : m_new));
       l_part *= alpha;
       m_run = m_new;
 #pragma unroll
@@ -144,11 +144,21 @@ __global__ __launch_bounds__(kThreads) void decode_attention_f32_kernel(
       }
     }
     const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+    // As weight_exp2; only waves with a result below 2^-126 (a masked token's
+    // counts) pay for the scaling.
+    float x[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      st[r] = fast_exp2(fmaf(st[r], kLog2e, -m_use));
-      l_part += st[r];
+    for (int r = 0; r < 4; ++r) x[r] = fmaf(st[r], kLog2e, -m_use);
+    if (__any(fminf(fminf(x[0], x[1]), fminf(x[2], x[3])) < -126.0f)) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[r] = exp2f(x[r]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st[r] = fast_exp2(x[r]);
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) l_part += st[r];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -195,7 +205,7 @@ __global__ __launch_bounds__(kThreads) void decode_attention_f32_kernel(
     float lsum = 0.0f, osum = 0.0f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      const float f = fast_exp2(sm_m[w][head] - mu);
+      const float f = weight_exp2<float>(sm_m[w][head] - mu);
       lsum += f * sm_l[w][head];
       osum += f * sm_o[w][head][d];
     }

@@ -78,7 +78,7 @@ __device__ __forceinline__ void merge_if_last(const float* part_o, const float* 
 #pragma unroll
         for (int k = 0; k < kFusedMergeUnroll; ++k) {
           if (k < nchunks) {
-            const float w = fast_exp2(m[o][k] - mu);  // exp2(-inf) = 0 for empty chunks
+            const float w = weight_exp2<T>(m[o][k] - mu);  // exp2(-inf) = 0 for empty chunks
             lsum[o] += w * l[o][k];
             acc[o] += w * (w != 0.0f ? v[o][k] : 0.0f);
           }
@@ -119,7 +119,7 @@ __device__ __forceinline__ void merge_if_last(const float* part_o, const float* 
 #pragma unroll
         for (int k = 0; k < kFusedMergeUnroll; ++k) {
           if (i0 + k < nchunks) {
-            const float w = fast_exp2(m[o][k] - mu);  // exp2(-inf) = 0 for empty chunks
+            const float w = weight_exp2<T>(m[o][k] - mu);  // exp2(-inf) = 0 for empty chunks
             lsum[o] += w * l[o][k];
             acc[o] += w * (w != 0.0f ? v[o][k] : 0.0f);
           }

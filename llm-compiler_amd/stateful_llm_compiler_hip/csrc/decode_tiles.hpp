@@ -63,6 +63,13 @@ __device__ __forceinline__ uint16_t bits_of(float f) {
 __device__ __forceinline__ float fast_exp2(float x) {
   return __builtin_amdgcn_exp2f(x);
 }
+// 2^x of fp32 attention: results below 2^-126 stay subnormal numbers, where the
+// instruction alone gives zero (a weight of 2^-130 on a value of 1e38 counts).
+template <typename T>
+__device__ __forceinline__ float weight_exp2(float x) {
+  if constexpr (std::is_same_v<T, float>) return exp2f(x);
+  return fast_exp2(x);
+}
 
 // LDS row stride (in 16-bit elements) of a staged V tile row.  The 4-element
 // pad makes the four token rows read by one transposed access land on disjoint

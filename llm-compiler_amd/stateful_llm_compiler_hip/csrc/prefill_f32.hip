@@ -230,20 +230,36 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_f32_kernel(
     if (__any(mx > m_run + kRescaleThreshold)) {
       mx = slc::max_xor32(slc::max_xor16(mx));
       const float m_new = fmaxf(m_run, mx);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
+      const float alpha = exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
       l_part *= alpha;
 #pragma unroll
       for (int db = 0; db < 4; ++db) acc[db] = acc[db] * alpha;
       m_run = m_new;
     }
     const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+    // Probabilities below 2^-126 stay subnormal numbers (exp2f), which only
+    // tiles that have one pay for; masked scores count.
+    float mn = st[0][0];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        st[kb][r] = __builtin_amdgcn_exp2f(fmaf(st[kb][r], kLog2e, -m_use));
-        l_part += st[kb][r];
-      }
+      for (int r = 0; r < 4; ++r) mn = fminf(mn, st[kb][r]);
+    if (__any(fmaf(mn, kLog2e, -m_use) < -126.0f)) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) st[kb][r] = exp2f(fmaf(st[kb][r], kLog2e, -m_use));
+    } else {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) st[kb][r] = __builtin_amdgcn_exp2f(fmaf(st[kb][r], kLog2e, -m_use));
+    }
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) l_part += st[kb][r];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll

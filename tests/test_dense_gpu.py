@@ -8,6 +8,8 @@ may differ by that rounding).  bf16 attention: 2e-2 absolute.
 
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -498,6 +500,23 @@ def test_prefill_grouped_kernel_scale(gpu, scale):
     actual, expected = _prefill_case(gpu, 2, 130, torch.bfloat16, 11, mask_kind="random", causal=True,
                                      scale=scale)
     assert_bf16_close(actual, expected)
+
+
+@pytest.mark.parametrize("order", ["online", "exact"])
+def test_prefill_fp32_subnormal_probability(gpu, order):
+    # exp(-89) = 2.2e-39, below the normal range, weighs a value of 1e38.
+    from stateful_llm_compiler_hip.backends import hip_prefill_attention
+
+    announce(f"prefill fp32 subnormal probability {order}")
+    g = generator(23)
+    q, k, v = (torch.randn(1, heads, 130, 64, generator=g) for heads in (4, 2, 2))
+    k.zero_()
+    mask = torch.full((1, 1, 130, 130), float("-inf"))
+    mask[..., 3], mask[..., 100] = 0, -89
+    v[:, :, 3], v[:, :, 100] = 0, 1e38
+    out = hip_prefill_attention(q.to(gpu), k.to(gpu), v.to(gpu), mask.to(gpu), scale=0.125, softmax_order=order)
+    # Two roundings of an exponent of 128, each at most 2^-17 ln 2.
+    assert (out.cpu().double() / (1e38 * math.exp(-89.0)) - 1).abs().max() <= 2 * 2.0**-17
 
 
 def _equal_fraction(actual, expected):

@@ -419,6 +419,25 @@ def test_decode_fp32_matrix_cores(gpu, batch, q_heads, kv_heads, head_dim, capac
     assert_fp32_close(actual[~empty], expected[~empty])
 
 
+@pytest.mark.parametrize("at", [1, 20, 150, 650])
+def test_decode_fp32_subnormal_probability(gpu, at):
+    # exp(-89) = 2.2e-39, below the normal range, weighs a value of 1e38: in the
+    # first token's step, in another wave's, in other chunks.
+    from stateful_llm_compiler_hip.backends import hip_decode_attention
+
+    announce(f"decode fp32 subnormal probability at token {at}")
+    g = generator(at)
+    q, k, v = (torch.randn(1, *shape, generator=g) for shape in ((4, 1, 64), (700, 2, 64), (700, 2, 64)))
+    k.zero_()
+    mask = torch.full((1, 1, 1, 700), float("-inf"))
+    mask[..., 0], mask[..., at] = 0, -89
+    v[:, 0], v[:, at] = 0, 1e38
+    out = hip_decode_attention(q.to(gpu), k.to(gpu), v.to(gpu), torch.tensor([700], device=gpu), mask.to(gpu),
+                               scale=0.125)
+    # Two roundings of an exponent of 128, each at most 2^-17 ln 2.
+    assert (out.cpu().double() / (1e38 * math.exp(-89.0)) - 1).abs().max() <= 2 * 2.0**-17
+
+
 def test_decode_fp32_mask_past_32_bit_chunks(gpu):
     # A mask far longer than the cache (one zero, expanded): a chunk of 2^31
     # tokens has no 32-bit end, and these 520 sequences take one chunk each.
