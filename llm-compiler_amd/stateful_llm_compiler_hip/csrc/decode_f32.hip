@@ -16,11 +16,16 @@
 //    token 4g + r, which is k-slot g of the A operand, so the probabilities
 //    never move; V rows are loaded 16 bytes per lane (row 4g + r, dims 4c ..
 //    4c + 3) and the MFMAs' columns are dims 4c + e.
+//  * A score's products are summed in chains of two MFMAs added in pairs: with
+//    two chains the result was up to 1.44 times as far from float64 as one wave
+//    per head with its sums across lanes (L64 D128 2.03e-7 against 1.40e-7, now
+//    1.35e-7; L300 D64 2.1e-7, 2.0e-7, now 1.7e-7; L32768 3.4e-7, 16e-7, now
+//    3.1e-7).  It costs 1 to 5 % of the time.
 //  * Sequences are split over about two workgroups per CU; partials merge in
 //    the last workgroup of each (batch, KV head), as in decode_kernel.hpp.
-// Measured against the wave-per-head kernel: B27 L9241 2614 -> 68 us (2.9 TB/s
-// of K and V, host launch included), B1 L32768 5074 -> 25, B16 L30000 D128
-// 11793 -> 181 (4.1 TB/s), B6 L247 61 -> 15 (host-bound).
+// Measured against the wave-per-head kernel (graphs of back-to-back calls, every
+// sequence at its full length): B27 L9241 2237 -> 57 us (4.5 TB/s of K and V), B1
+// L32768 7371 -> 28, B16 L30000 D128 12262 -> 204 (4.8 TB/s), B6 L247 35 -> 8.4.
 #include "common.hpp"
 #include "decode_kernel.hpp"
 
@@ -111,18 +116,23 @@ __global__ __launch_bounds__(kThreads) void decode_attention_f32_kernel(
     for (int e = 0; e < 4; ++e) acc[h][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   auto compute = [&](int t0, const Step& s) {
-    f32x4_t st = f32x4_t{0.f, 0.f, 0.f, 0.f}, st2 = st;  // two chains
+    // Chains of two MFMAs, added in pairs: a long chain rounds its partial sums
+    // one after the other.
+    f32x4_t st = f32x4_t{0.f, 0.f, 0.f, 0.f}, part[2 * KK];
 #pragma unroll
-    for (int kk = 0; kk < KK; kk += 2)
+    for (int kk = 0; kk < KK; ++kk) {
+      part[2 * kk] = mfma4(s.k[kk][1], qv[kk][1], mfma4(s.k[kk][0], qv[kk][0], st));
+      part[2 * kk + 1] = mfma4(s.k[kk][3], qv[kk][3], mfma4(s.k[kk][2], qv[kk][2], st));
+    }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        st = mfma4(s.k[kk][e], qv[kk][e], st);
-        st2 = mfma4(s.k[kk + 1][e], qv[kk + 1][e], st2);
-      }
+    for (int n = KK; n > 0; n /= 2)
+#pragma unroll
+      for (int i = 0; i < n; ++i) part[i] = part[2 * i] + part[2 * i + 1];
+    st = part[0];
     float mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      float v = (st[r] + st2[r]) * scale;
+      float v = st[r] * scale;
       if constexpr (MK != 0) v += s.mk[r];
       st[r] = t0 + 4 * g + r < end ? v : -INFINITY;
       mx = fmaxf(mx, st[r]);

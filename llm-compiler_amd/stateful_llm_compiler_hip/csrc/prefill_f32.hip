@@ -9,8 +9,9 @@
 //
 // What bounds it: the matrix cores.  v_mfma_f32_16x16x4_f32 does 64 FLOP per
 // cycle and SIMD, so a wave's 128 MFMAs on a 64-key tile take 4096 cycles
-// against about 900 of softmax VALU and 1024 of LDS reads for its workgroup:
-// memory and LDS hide behind them with two workgroups per CU.
+// against about 1500 of VALU (softmax, and the sums that keep the error below
+// one chain's) and 1024 of LDS reads for its workgroup: memory and LDS hide
+// behind them with two workgroups per CU.
 //  * A workgroup is 4 waves of 16 queries each of one query head; 64-key K and
 //    V tiles (16 KB each) are double-buffered in LDS, filled by direct loads.
 //  * S^T[key, query] = K . Q^T: lane (row c, group g) reads the 16-byte chunk
@@ -25,9 +26,15 @@
 //  * Key tiles that the mask's classes rule out are not visited, tiles of the
 //    causal pattern are masked from the indices, and only the rest read their
 //    mask, element by element (any strides), under the score MFMAs.
-// Measured against one wave per query: B8 T512 padded causal mask 4548 -> 53
-// us, B6 T1000 causal 3643 -> 105 us (102 TFLOP/s of the causal products; a
-// large fp32 library product reaches 153 on this card), B5 T125 254 -> 19.
+//  * A score is eight chains of two MFMAs added in pairs, and a tile's sums over
+//    its keys are added to the running ones once: a single chain of 64 products
+//    and one over all keys were up to 1.44 times as far from float64 as one wave
+//    per query with its sums across lanes (16 tokens 1.21e-7 against 0.84e-7,
+//    now 0.81e-7; 200 tokens 2.3e-7 against 1.8e-7, now 1.4e-7; 1000 tokens
+//    3.3e-7, 3.2e-7, now 1.6e-7).  It costs 8 to 11 % of the time.
+// Measured against one wave per query: B8 T512 padded causal mask 2930 -> 58
+// us, B6 T1000 causal 3670 -> 117 us (92 TFLOP/s of the causal products; a
+// large fp32 library product reaches 153 on this card), B1 T64 29 -> 6.4.
 #include <algorithm>
 
 #include "common.hpp"
@@ -187,19 +194,20 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_f32_kernel(
         }
       }
     }
+    // Eight chains of two MFMAs per score, added in pairs: one chain of sixteen
+    // rounds 64 partial sums one after the other.
     f32x4_t st[4];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) st[kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int kb = 0; kb < 4; ++kb) {
+      f32x4_t part[8];
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      f32x4_t ka[4];
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-        ka[kb] = *reinterpret_cast<const f32x4_t*>(tile + k_read[kk] + 16 * kb * kRow);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) st[kb] = mfma4(ka[kb][j], qv[kk][j], st[kb]);
+      for (int kk = 0; kk < 4; ++kk) {
+        const f32x4_t ka = *reinterpret_cast<const f32x4_t*>(tile + k_read[kk] + 16 * kb * kRow);
+        const f32x4_t z = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        part[2 * kk] = mfma4(ka[1], qv[kk][1], mfma4(ka[0], qv[kk][0], z));
+        part[2 * kk + 1] = mfma4(ka[3], qv[kk][3], mfma4(ka[2], qv[kk][2], z));
+      }
+      st[kb] = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
     }
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
@@ -256,10 +264,16 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_f32_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) st[kb][r] = __builtin_amdgcn_exp2f(fmaf(st[kb][r], kLog2e, -m_use));
     }
+    // The tile's own sums first, then one addition each to the running ones.
+    float l_tile = 0.0f;
+    f32x4_t pv[4];
+#pragma unroll
+    for (int db = 0; db < 4; ++db) pv[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) l_part += st[kb][r];
+      for (int r = 0; r < 4; ++r) l_tile += st[kb][r];
+    l_part += l_tile;
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
@@ -267,8 +281,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void prefill_attention_f32_kernel(
 #pragma unroll
         for (int db = 0; db < 4; ++db) {
           const float v = *reinterpret_cast<const float*>(tile + v_read[db] + (16 * kb + r) * kRow);
-          acc[db] = mfma4(v, st[kb][r], acc[db]);
+          pv[db] = mfma4(v, st[kb][r], pv[db]);
         }
+#pragma unroll
+    for (int db = 0; db < 4; ++db) acc[db] = acc[db] + pv[db];
   }
 
   // The row sum over the 4 lane groups; an empty row is 0 * inf = NaN, as the

@@ -69,3 +69,30 @@ def assert_bitwise_equal(actual: torch.Tensor, expected: torch.Tensor) -> None:
     b = expected.view(width)
     differ = (a != b).sum().item()
     assert differ == 0, f"{differ} of {a.numel()} elements differ bitwise"
+
+
+def attention_exact(query, key, value, bias, scale):
+    """Float64 attention of [B, H, T, D] queries over [B, KVH, S, D] keys and values."""
+
+    groups = query.shape[1] // key.shape[1]
+    key, value = (t.double().repeat_interleave(groups, dim=1) for t in (key, value))
+    return torch.softmax(query.double() @ key.transpose(-1, -2) * scale + bias.double(), -1) @ value
+
+
+def attention_in_chains(query, key, value, bias, scale):
+    """The same in fp32 with every sum as one chain in index order."""
+
+    groups = query.shape[1] // key.shape[1]
+    key, value = (t.repeat_interleave(groups, dim=1) for t in (key, value))
+    scores = torch.zeros(*query.shape[:3], key.shape[2])
+    for d in range(query.shape[-1]):
+        scores = scores + query[..., d, None] * key[..., None, :, d]
+    probabilities = torch.softmax(scores * scale + bias, -1)
+    out = torch.zeros_like(query)
+    for j in range(key.shape[2]):
+        out = out + probabilities[..., j, None] * value[..., None, j, :]
+    return out
+
+
+def relative_error(actual: torch.Tensor, exact: torch.Tensor) -> float:
+    return float((actual.double().cpu() - exact).norm() / exact.norm())

@@ -13,7 +13,15 @@ import math
 import pytest
 import torch
 
-from helpers import announce, assert_bf16_close, assert_fp32_close, generator
+from helpers import (
+    announce,
+    assert_bf16_close,
+    assert_fp32_close,
+    attention_exact,
+    attention_in_chains,
+    generator,
+    relative_error,
+)
 from oracle import kernels as ref
 
 pytestmark = pytest.mark.gpu
@@ -517,6 +525,24 @@ def test_prefill_fp32_subnormal_probability(gpu, order):
     out = hip_prefill_attention(q.to(gpu), k.to(gpu), v.to(gpu), mask.to(gpu), scale=0.125, softmax_order=order)
     # Two roundings of an exponent of 128, each at most 2^-17 ln 2.
     assert (out.cpu().double() / (1e38 * math.exp(-89.0)) - 1).abs().max() <= 2 * 2.0**-17
+
+
+@pytest.mark.parametrize("tokens", [16, 65, 200])
+def test_prefill_fp32_error_below_single_chains(gpu, tokens):
+    """The squared error of a chain of n fp32 additions grows as n^2 / 2: 64
+    products in one chain 2048, in eight of 8 added in pairs 448, and the sums
+    over the keys of a 64-key tile are added once each.  So the kernel stays
+    well below one chain per sum (0.6 to 0.7 of its error; 1.0 with a chain)."""
+
+    from stateful_llm_compiler_hip.backends import hip_prefill_attention
+
+    announce(f"prefill fp32 error T={tokens}")
+    g = generator(tokens)
+    q, k, v = (torch.randn(2, heads, tokens, 64, generator=g) for heads in (14, 2, 2))
+    bias = torch.zeros(tokens, tokens).masked_fill(torch.ones(tokens, tokens).triu(1).bool(), float("-inf"))
+    exact = attention_exact(q, k, v, bias, 0.125)
+    out = hip_prefill_attention(q.to(gpu), k.to(gpu), v.to(gpu), None, scale=0.125, causal=True)
+    assert relative_error(out, exact) <= 0.8 * relative_error(attention_in_chains(q, k, v, bias, 0.125), exact)
 
 
 def _equal_fraction(actual, expected):
