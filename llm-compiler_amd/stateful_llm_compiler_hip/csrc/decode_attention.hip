@@ -204,7 +204,7 @@ Plan plan_call(int dtype, int64_t batch, int64_t q_heads, int64_t kv_heads,
     p.chunk = mask_len;
     p.nchunks = 1;
   } else {
-    p.chunk = choose_chunk(batch, kv_heads, mask_len, split_tokens);
+    p.chunk = choose_chunk(batch, kv_heads, head_dim, mask_len, split_tokens);
     p.nchunks = slc_host::ceil_div(mask_len, p.chunk);
   }
   p.need = partial_bytes(batch, q_heads, head_dim, p.nchunks);

@@ -873,7 +873,7 @@ __global__ __launch_bounds__(256) void decode_attention_merge_kernel(
 
 // Any dtype / head_dim <= 256 / any group size: one workgroup per
 // (batch, query head), each wave takes every 4th token and reduces q.k with
-// shuffles.  Used for fp32 and for shapes the MFMA kernel does not cover.
+// shuffles.  Used for shapes the MFMA kernels do not cover.
 // EXACT: the reference's softmax order (normalise, round, then P.V) in two
 // passes over the keys: the first forms the row max and sum, the second
 // recomputes each score and weighs V with its normalised, rounded probability.
@@ -986,34 +986,62 @@ bool mfma_eligible(int dtype, int64_t head_dim, int64_t groups) {
 }
 
 // Sequence chunk of the split-sequence grid, a multiple of the workgroup's
-// 128-token sweep.  A workgroup takes about 7 ns per token of its chunk, a
-// split about 4 us for publishing and merging and 0.2 us per chunk more, and
-// past one workgroup per CU (256 on MI355X) every further release write-back
-// costs more than it saves.  So (graphs of back-to-back calls, microseconds):
-//  * one chunk where splitting gains less than the merge: masks up to 640
-//    tokens (B1 L512 8.0 -> 6.0, B48 L600 11.4 -> 8.2), and up to 1024 where
-//    the grid leaves two chunks at most (B64 L1024 12.9 -> 11.8);
+// 128-token sweep.  A workgroup takes about 7.3 ns per token of its chunk at
+// head_dim 64 and 14.5 at 128, a split about 3 us for publishing and merging, a
+// microsecond or more of them per batch of eight chunks that the merge loads at
+// once, and past one workgroup per CU (256 on MI355X) every further release
+// write-back costs more than it saves.  The rule sees the mask, not the lengths,
+// which are on the device.  Graphs of back-to-back calls, us, lengths between two
+// thirds of the mask and all of it, and in brackets up to 15 % of it:
+//  * one chunk for masks up to 640 tokens, 512 at head_dim 128, and up to 1024
+//    where the grid leaves two chunks at most.  Splitting gains less there than the merge costs at
+//    head_dim 64 (L512 B16 one 7.8 [5.1], two 8.6 [7.2]; B64 L1024 12.0 [5.8],
+//    two 13.5 [9.9]).  At 128 it depends on the lengths: full caches are better
+//    split (two KV heads, B16 L512 one 11.8 [6.4], two 11.1 [8.3]; L640 13.6 [6.5],
+//    three 11.5 [8.9]; B64 L1024 20.4 [7.8], two 18.9 [11.4]), emptier ones are
+//    not: over 15, 75 and 100 % one chunk is 5 to 12 % less in sum at 512 and 1024
+//    and no less at 640;
 //  * else equal chunks of at least 256 tokens, at most one workgroup per CU
 //    (B20 L17963 D128: six chunks of 3072 tokens 68, five of 4096 80);
-//  * and chunk^2 >= 16 mask_len, which balances the chunk against the merge
-//    for few long sequences (B1 L32768: 128 chunks of 256 34.8, 32 of 1024
-//    19.3; B1 L16384 22.3 -> 16.4).
-int64_t choose_chunk(int64_t batch, int64_t kv_heads, int64_t mask_len,
+//  * chunk^2 >= 16 mask_len, which balances the chunk against the merge for few
+//    long sequences (B1 L32768: 128 chunks of 256 37.8, 32 of 1024 20.1; B1 L16384
+//    22.1 -> 16.4).  A short sequence in a long cache pays that merge all the same:
+//    every chunk past its length publishes an empty part;
+//  * at head_dim 64 chunks of 512 tokens rather than a grid that leaves hardly a
+//    CU free (B32 L1500: 512 x 3 10.9, 384 x 4 12.4, all 256 CUs; but B24 L1800:
+//    384 x 5, 240 CUs, 11.0, 512 x 4 12.1);
+//  * and no last batch of the merge begun where longer chunks cost less (B5
+//    L8192: 512 x 16 13.9, 384 x 22 15.2; B24 L8192, one KV head: 1024 x 8 17.0,
+//    896 x 10 18.4).
+int64_t choose_chunk(int64_t batch, int64_t kv_heads, int64_t head_dim, int64_t mask_len,
                      int64_t split_tokens) {
   const int64_t sweep = kWaves * kTile;
   auto sweeps = [&](int64_t tokens) { return slc_host::ceil_div(tokens, sweep) * sweep; };
+  auto chunks = [&](int64_t tokens) { return slc_host::ceil_div(mask_len, tokens); };
   int64_t chunk;
   if (split_tokens > 0) {
     chunk = sweeps(split_tokens);
   } else {
-    const int64_t most = std::max<int64_t>(1, 256 / std::max<int64_t>(1, batch * kv_heads));
-    if (mask_len <= 640 || (most <= 2 && mask_len <= 1024)) {
+    const bool wide = head_dim > 64;
+    const int64_t pairs = std::max<int64_t>(1, batch * kv_heads);
+    const int64_t most = std::max<int64_t>(1, 256 / pairs);
+    if (mask_len <= (wide ? 512 : 640) || (most <= 2 && mask_len <= 1024)) {
       chunk = sweeps(mask_len);
     } else {
       chunk = std::max<int64_t>(256, sweeps(slc_host::ceil_div(mask_len, most)));
       while (chunk * chunk < 16 * mask_len) chunk += sweep;
+      while (!wide && chunk < 512 && pairs * chunks(chunk) > 240) chunk += sweep;
       // Equal chunks: as many as that leaves, no longer than they need be.
-      chunk = sweeps(slc_host::ceil_div(mask_len, slc_host::ceil_div(mask_len, chunk)));
+      const int64_t n = chunks(chunk);
+      chunk = sweeps(slc_host::ceil_div(mask_len, n));
+      if (n > 8 && n % 8 != 0) {
+        // Nanoseconds of a chunk's tokens and of the merge's batches.
+        auto cost = [&](int64_t tokens) {
+          return tokens * (wide ? 145 : 73) / 10 + slc_host::ceil_div(chunks(tokens), 8) * (wide ? 1000 : 1400);
+        };
+        const int64_t longer = sweeps(slc_host::ceil_div(mask_len, n / 8 * 8));
+        if (cost(longer) < cost(chunk)) chunk = longer;
+      }
     }
   }
   // The merge keeps every chunk's weight of a (batch, kv-head) in LDS.

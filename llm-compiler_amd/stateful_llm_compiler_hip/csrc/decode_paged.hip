@@ -198,7 +198,7 @@ extern "C" int slc_hip_paged_decode_attention(
     chunk = mask_len;
     nchunks = 1;
   } else {
-    chunk = choose_chunk(batch, kv_heads, mask_len, split_tokens > 0 ? split_tokens : 0);
+    chunk = choose_chunk(batch, kv_heads, head_dim, mask_len, split_tokens > 0 ? split_tokens : 0);
     nchunks = slc_host::ceil_div(mask_len, chunk);
   }
   const int64_t need = partial_bytes(batch, q_heads, head_dim, nchunks);
@@ -325,7 +325,7 @@ extern "C" int slc_hip_paged_rope_decode_attention(
     chunk = mask_len;
     nchunks = 1;
   } else {
-    chunk = choose_chunk(batch, kv_heads, mask_len, 0);
+    chunk = choose_chunk(batch, kv_heads, head_dim, mask_len, 0);
     nchunks = slc_host::ceil_div(mask_len, chunk);
   }
   const int64_t need = partial_bytes(batch, q_heads, head_dim, nchunks);

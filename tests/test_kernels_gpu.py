@@ -175,6 +175,19 @@ def test_decode_attention_config2_bf16(gpu, batch, max_len, split):
     assert_bf16_close(actual, expected)
 
 
+@pytest.mark.parametrize("batch,q_heads,kv_heads,head_dim,max_len", [
+    (32, 14, 2, 64, 1500), (5, 14, 2, 64, 8192), (24, 8, 1, 64, 8192), (3, 8, 2, 128, 12000),
+])
+def test_decode_attention_chosen_chunks(gpu, batch, q_heads, kv_heads, head_dim, max_len):
+    # Chunk counts of the full-grid and whole-merge-batch rules; nearly empty,
+    # half full and full caches.
+    announce(f"decode bf16 B={batch} KVH={kv_heads} D={head_dim} L={max_len}")
+    lengths = [(1, max_len // 2, max_len)[i % 3] for i in range(batch)]
+    actual, expected = _decode_case(gpu, batch, q_heads, kv_heads, head_dim, max_len, lengths,
+                                    torch.bfloat16, batch + max_len)
+    assert_bf16_close(actual, expected)
+
+
 @pytest.mark.parametrize("split", [0, SPLIT_BALANCED])
 @pytest.mark.parametrize("batch", [1, 8, 32, 64])
 def test_decode_attention_config2_bf16_long(gpu, batch, split):

@@ -69,6 +69,21 @@ def test_argument_checks_fail_without_touching_a_device():
     assert lib.slc_hip_argmax_workspace_size(8) == 8 * 64 * 12
 
 
+@pytest.mark.parametrize("batch,kv_heads,head_dim,mask_len,chunks", [
+    (16, 2, 64, 640, 1), (16, 2, 64, 641, 3),          # one chunk up to 640 tokens,
+    (16, 2, 128, 512, 1), (16, 2, 128, 513, 3),        # up to 512 of 128 features
+    (64, 2, 128, 1024, 1), (64, 2, 128, 1025, 2),      # up to 1024 where two are the most
+    (32, 2, 64, 1500, 3), (32, 2, 128, 1500, 4),       # 512-token chunks past 240 workgroups
+    (5, 2, 64, 8192, 16), (24, 1, 64, 8192, 8),        # whole batches of eight in the merge
+    (20, 2, 128, 17963, 6),                            # at most one workgroup per CU
+])
+def test_decode_chunk_counts(batch, kv_heads, head_dim, mask_len, chunks):
+    # The workspace holds D + 2 floats for each chunk of each head, none unsplit.
+    size = _native.library().slc_hip_decode_attention_workspace_size(
+        batch, 8, head_dim, mask_len, kv_heads, 2, 0)
+    assert size == (0 if chunks == 1 else batch * 8 * chunks * (head_dim + 2) * 4)
+
+
 @pytest.mark.parametrize("stages,compiles", [(2, True), (3, False)])
 def test_masked_prefill_takes_two_ring_stages_only(stages, compiles):
     # A deeper ring's wait counts loads that an element-loaded mask tile does
