@@ -442,14 +442,29 @@ int linear_f32(const float* x, const float* w, const float* bias, float* y, int 
       int64_t{128} * K * 4 >= (int64_t{1} << 31))
     return SLC_ERR_UNSUPPORTED;
   const int64_t cus = device_cu_count();
+  const int64_t blocks16 = ceil_div(N, 16) * ceil_div(M, 16);
+  // Short K leaves these kernels little but their start and their epilogue: the
+  // generic kernel takes K below 64 (K32: 16 rows N4864 10.5 us here, 2.8 there;
+  // 4096 rows N16384 K4 588 | 137) except large grids of whole k-tiles (4096 rows
+  // N4864 K32 0.4 of its time), and up to 92 many rows past the ring's k-tiles.
+  if (K < 64 && (K % kBK != 0 || M <= 16 || blocks16 <= 8 * cus)) return SLC_ERR_UNSUPPORTED;
+  if (K < 96 && K % kBK != 0 && M > 16 && blocks16 > 2 * cus) return SLC_ERR_UNSUPPORTED;
   if (M <= 16) {
-    // One round of workgroups of 4, 8 or 20 features each, while that covers N.
-    if (N <= 4 * cus) return launch_few<1, 16, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-    if (N <= 8 * cus) return launch_few<2, 16, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
-    if (N <= 20 * cus) return launch_few<5, 8, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
+    // One round of workgroups of 4, 8 or 20 features each, while that covers N
+    // and K is long enough for the sums over the waves at the end, which grow
+    // with the features and rows (16 rows N4864: K256 10.8 us, the generic kernel
+    // 8.4, 16-feature workgroups 4.2; K384 11.3 | 11.5 | 5.5, with three times the
+    // error; 16 rows N1500 K128 6.6 | 4.9 | 3.3; 8 rows N4864 K128 6.5 | 5.1 | 3.3).
+    const int rows = M <= 4 ? 0 : (M <= 8 ? 1 : 2);
+    constexpr int kLeast[3][3] = {{64, 96, 128}, {96, 128, 256}, {128, 256, 384}};
+    if (N <= 4 * cus && K >= kLeast[0][rows])
+      return launch_few<1, 16, 2>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
+    if (N > 4 * cus && N <= 8 * cus && K >= kLeast[1][rows])
+      return launch_few<2, 16, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
+    if (N > 8 * cus && N <= 20 * cus && K >= kLeast[2][rows])
+      return launch_few<5, 8, 1>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
     return launch_rows<1, 4, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);
   }
-  const int64_t blocks16 = ceil_div(N, 16) * ceil_div(M, 16);
   if (K % kBK != 0 || blocks16 <= 2 * cus) {
     if (M > 65535 * 16) return SLC_ERR_UNSUPPORTED;
     if (blocks16 <= cus) return launch_rows<1, 16, 4>(x, w, bias, y, M, N, K, x_rs, y_rs, s);

@@ -373,6 +373,15 @@ def test_linear_fp32_matrix_cores(gpu, rows, n, k, bias):
     assert (actual - exact).norm() <= 2 * k**0.5 * 2.0**-24 * terms.norm()
 
 
+@pytest.mark.parametrize("rows", [1, 4, 8, 16, 17, 300])
+@pytest.mark.parametrize("n,k", [
+    (130, 48), (5000, 32), (20000, 32), (5000, 92), (5000, 96), (5000, 100),  # generic below, K % 32 past two rounds
+    (700, 64), (700, 128), (1500, 96), (1500, 256), (4864, 128), (4864, 256), (4864, 384),  # features per workgroup
+])
+def test_linear_fp32_short_k(gpu, rows, n, k):
+    test_linear_fp32_matrix_cores(gpu, rows, n, k, rows % 2 == 0)
+
+
 # -------------------------------------------------------- prefill attention
 
 
