@@ -151,8 +151,10 @@ __device__ __forceinline__ uint2 lds_read_tr(const unsigned char* p) {
 // no data but keep every tile's load count equal); pass 2 recomputes the
 // scores and weighs V with exp(score - max) / sum rounded to the I/O dtype,
 // so the rounding applies to the normalised probability as in the reference.
-template <typename T, int G, int MK, bool CAUSAL, bool POW2, bool EXACT, int QB>
-__global__ __launch_bounds__((G + 1) * 64, QB <= 2 ? 4 : 1) void prefill_attention_v2_kernel(
+// WAVES: the waves per SIMD its registers have to leave room for (see launch_v2).
+template <typename T, int G, int MK, bool CAUSAL, bool POW2, bool EXACT, int QB,
+          int WAVES = QB <= 2 ? 4 : 1>
+__global__ __launch_bounds__((G + 1) * 64, WAVES) void prefill_attention_v2_kernel(
     const T* __restrict__ query, const T* __restrict__ key, const T* __restrict__ value,
     const void* __restrict__ mask, T* __restrict__ output, int tokens, int kv_heads,
     int64_t q_sb, int64_t q_sh, int64_t q_st, int64_t k_sb, int64_t k_sh, int64_t k_st,
@@ -654,6 +656,16 @@ int launch_v2(const void* q, const void* k, const void* v, const void* mask, voi
                               : prefill_attention_v2_kernel<T, G, MK, CAUSAL, false, true, QB>)
                       : (pow2 ? prefill_attention_v2_kernel<T, G, MK, CAUSAL, true, false, QB>
                               : prefill_attention_v2_kernel<T, G, MK, CAUSAL, false, false, QB>);
+  if constexpr (G == 8 && MK == 0 && QB == 1) {
+    // Nine waves per workgroup: with the 82 to 86 registers that the exact order
+    // takes when free to, two fit a CU, with 72 three.  Short grids gain from the
+    // registers (B1 T1024, four heads per workgroup: 17.5 | 21.6 us), grids past
+    // two workgroups per CU from the third (8 heads, 4 KV heads: B4 T1024 51 | 44,
+    // B8 T512 33 | 28; 1 KV head: B3 T4096 139 | 122).
+    if (exact && int64_t{grid.x} * grid.y * grid.z > 2 * int64_t{slc_host::device_cu_count()})
+      kernel = pow2 ? prefill_attention_v2_kernel<T, G, MK, CAUSAL, true, true, QB, 7>
+                    : prefill_attention_v2_kernel<T, G, MK, CAUSAL, false, true, QB, 7>;
+  }
   hipLaunchKernelGGL(kernel, grid, dim3((G + 1) * 64), 0,
                      stream, static_cast<const T*>(q), static_cast<const T*>(k),
                      static_cast<const T*>(v), mask, static_cast<T*>(out), tokens, kv_heads,

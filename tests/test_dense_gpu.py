@@ -428,6 +428,19 @@ def test_prefill_causal_flag_bf16(gpu, batch, tokens):
     assert_bf16_close(actual, expected)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("causal,scale", [(True, None), (True, 0.11), (False, None)])
+@pytest.mark.parametrize("batch,tokens", [(9, 896), (9, 901)])
+def test_prefill_exact_eight_heads_grids(gpu, batch, tokens, causal, scale, dtype):
+    """Eight heads per KV head without a mask: 504 and 513 workgroups, on both
+    sides of two per CU."""
+
+    announce(f"prefill exact {dtype} B={batch} T={tokens} causal={causal} scale={scale}")
+    actual, expected = _prefill_case(gpu, batch, tokens, dtype, tokens, mask_kind="none", causal=causal,
+                                     q_heads=8, kv_heads=1, scale=scale, softmax_order="exact")
+    assert_bf16_close(actual, expected)
+
+
 @pytest.mark.parametrize("batch,kind", [(2, "causal"), (8, "none")])
 def test_prefill_bench_shapes_bf16(gpu, batch, kind):
     """Config 4's longest prompts (T = 4096) at the shapes the bench times:
