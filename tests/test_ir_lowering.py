@@ -352,6 +352,26 @@ def test_committed_mi355x_profile_plans_the_measured_winners():
     assert choose_variant(split, 32 * 8192).variant == "fixed"
 
 
+def test_committed_mi355x_profile_samples_every_linear_tile():
+    """A tile that the library's own rule takes but the profile lacks would be
+    planned away: the large linears run on the persistent s256x128."""
+
+    import json
+    from pathlib import Path
+
+    import stateful_llm_compiler_hip
+    from stateful_llm_compiler_hip.profile_variants import LINEAR_ROWS, LINEAR_SHAPES, LINEAR_VARIANTS
+
+    path = Path(stateful_llm_compiler_hip.__file__).parent / "profiles" / "mi355x.json"
+    samples = json.loads(path.read_text(encoding="utf-8"))["linear"]
+    assert {(s["rows"], s["out_features"], s["in_features"]) for s in samples} == {
+        (m, n, k) for n, k in LINEAR_SHAPES for m in LINEAR_ROWS}
+    assert all(set(s["hip_variants"]) == set(LINEAR_VARIANTS) for s in samples)
+    plan = KernelProfile.load(path).plan("linear", out_features=4864, in_features=896, dtype="bf16")
+    for rows in (4096, 8192, 20000, 32768):
+        assert choose_variant(plan, rows).variant == "s256x128"
+
+
 def test_plan_changes_the_variant_the_executor_launches(monkeypatch):
     """The plan's choice reaches the HIP wrapper's launch argument (and from
     there the C ABI's waves_per_row / split_tokens) and the lowering trace."""
