@@ -211,6 +211,44 @@ def test_config5_fp32_fast_mode(gpu):
             raise AssertionError(f"{what}: {error}") from None
 
 
+def _model_error(gpu, monkeypatch, batch, tokens, seed):
+    """Relative and largest error of a two-layer fp32 prefill (capacity 2048)
+    against the eager model in float64: of the logits, and of K and V over the
+    written cache slots, the largest in units of their root mean square."""
+
+    config = Qwen2Config(num_layers=2, vocab_size=1024)
+    weights = init_weights(config, seed=seed, dtype=torch.float32, device=gpu, draw_on_device=True)
+    ids = torch.randint(0, config.vocab_size, (batch, tokens), generator=torch.Generator().manual_seed(seed))
+    mask, pos = causal_prefill_mask(batch, tokens), torch.arange(tokens).view(1, -1).expand(batch, -1).contiguous()
+    with monkeypatch.context() as patch:
+        # The eager model rounds its norms, rotations and softmax with .float().
+        patch.setattr(torch.Tensor, "float", torch.Tensor.double)
+        exact, cache = EagerQwen2(config, {k: w.cpu().double() for k, w in weights.items()}).prefill(ids, mask, pos)
+    rt = Qwen2Runtime(config, weights, capacity=CAPACITY, dtype=torch.float32, device=str(gpu))
+    logits, state = rt.prefill(ids.to(gpu), mask.to(gpu), pos.to(gpu))
+    torch.cuda.synchronize()
+    keys, values = ([t[:, :tokens].transpose(1, 2) for t in side] for side in (state.keys, state.values))
+    pairs = {"logits": (logits, exact), "keys": (torch.stack(keys), torch.stack([k for k, _ in cache])),
+             "values": (torch.stack(values), torch.stack([v for _, v in cache]))}
+    errors = {}
+    for what, (a, e) in pairs.items():
+        d = a.cpu().double() - e
+        errors[what] = (float(d.norm() / e.norm()), float(d.abs().max() / e.pow(2).mean().sqrt()))
+    return errors
+
+
+@pytest.mark.parametrize("batch,tokens", [(1, 6), (2, 37)])
+def test_fp32_prefill_error_in_a_nearly_empty_cache(gpu, monkeypatch, batch, tokens):
+    announce(f"fp32 two-layer prefill of {batch} x {tokens} in {CAPACITY} slots against float64")
+    errors = _model_error(gpu, monkeypatch, batch, tokens, seed=tokens)
+    _record(f"fp32_prefill_{batch}x{tokens}", errors)
+    # Linears that add all of K in one fp32 chain reach 1.9e-6 and 2.0e-6 on the
+    # logits, largest 8.0e-6 and 8.8e-6 of the root mean square; with K in
+    # several chains 3.4e-7 and 1.0e-6, largest 1.3e-6 and 4.5e-6.
+    for what, (relative, largest) in errors.items():
+        assert relative <= 1.5e-6 and largest <= 6e-6, (what, relative, largest)
+
+
 # Bars for fast mode over the full 128-step run: 1.5x the GEMM-rounding
 # yardstick that test_config5_fast_mode measures on this model (eager moves
 # its logits by 0.070 and its K/V by 0.0625 when only its linears' rounding
