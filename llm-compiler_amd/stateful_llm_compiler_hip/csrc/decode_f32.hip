@@ -245,8 +245,10 @@ bool decode_f32_eligible(int64_t head_dim, int64_t groups) {
 
 int64_t decode_f32_chunks(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
                           int64_t mask_len) {
-  // Two workgroups per CU, at least two sweeps of tokens each, and partials
-  // of at most 8 MiB (what the no-allocation entry point holds).
+  // Two workgroups for each of MI355X's 256 CUs, at least two sweeps of tokens
+  // each, and partials of at most 8 MiB (what the no-allocation entry point
+  // holds).  The count is a constant, as in choose_chunk: it sizes the caller's
+  // workspace, which is asked for without a device.
   int64_t n = std::min<int64_t>(512 / std::max<int64_t>(1, batch * kv_heads),
                                 ceil_div(mask_len, 2 * kSweepF32));
   n = std::min<int64_t>(n, 64);

@@ -668,25 +668,27 @@ __device__ __forceinline__ void xcd_tile_of(int id, int n_tiles, int m_tiles, in
   n_blk = (t % span) / gm;
 }
 
-// Persistent form of the 256 x 128 ring tile, for grids several rounds deep.
+// Swizzle of the persistent kernel's W tile: the 16 rows of a fragment that it
+// reads are four runs of four, eight apart, so the key takes row bits 0, 1 and 3.
+__device__ __forceinline__ int w_key(int row) { return (row & 3) | ((row >> 1) & 4); }
+
+// Persistent form of the 256 x 128 ring tile, for every plain grid of such tiles
+// and for deep gate/up grids (stream_grid).
 // One workgroup per CU walks the output tiles id, id + grid, ...; its
 // producer waves stream k-tiles into the 3-stage ring without a break at tile
 // boundaries, so the first k-tiles of the next output tile land while the
 // consumers finish the current one and write it out.  The consumers multiply
-// with the operands swapped (W rows as the MFMA A operand, X rows as B): an
-// accumulator lane then holds four consecutive output features of one row,
-// which it stores with one 8-byte store straight from registers -- the ring
-// is never needed for staging the output.  Each output accumulates its k
+// with the operands swapped (W rows as the MFMA A operand, X rows as B), and the
+// W rows of two fragments are interleaved in runs of four: a lane's accumulators
+// of the pair then hold eight consecutive output features of one row, which it
+// stores with one 16-byte store straight from registers -- the ring is never
+// needed for staging the output.  Each output accumulates its k
 // range in the ring kernel's order (same fragments, same 32-k MFMA steps; a
 // product of two bf16 values does not depend on which operand slot holds
 // which), so both kernels give the same bits.
 // DUAL: each 128-row W stage holds 64 gate rows then 64 up rows; consumer
 // wave wn takes gate and up rows of the same 32 features (fragments 0-1 gate,
 // 2-3 up), so the SwiGLU pairs meet in one lane.
-// The W tile's own swizzle: the 16 rows of a fragment read below are four runs
-// of four, eight apart, so the key takes row bits 0, 1 and 3.
-__device__ __forceinline__ int w_key(int row) { return (row & 3) | ((row >> 1) & 4); }
-
 template <typename T, bool DUAL>
 __global__ __launch_bounds__(12 * 64) void linear_stream_kernel(
     const T* __restrict__ x, const T* __restrict__ w_arg, const T* __restrict__ bias_arg,
@@ -983,8 +985,8 @@ int launch_ring(const void* x, const void* w, const void* bias, void* y, int M, 
 // when there are fewer tiles.  kNoResidualPath where the shape does not fit.
 // The library launches it for every plain linear of 256 x 128 tiles: its stores
 // drain under the next tile's MFMAs, where the ring kernel's workgroups end with
-// them (M4096 N4864 K896 43.9 -> 40.1 us, M8192 73.9 -> 66.3, M32768 341 -> 308,
-// vocabulary head of 4096 rows 1270 -> 1202), and with one tile per workgroup it
+// them (M4096 N4864 K896 43.9 -> 40.1 us, M8192 73.9 -> 66.3, M32768 304 -> 280,
+// vocabulary head of 4096 rows 1262 -> 1190), and with one tile per workgroup it
 // is ahead by its wider stores from registers (M8192 N896 K4864 63.9 -> 62.2, K896
 // 17.9 -> 17.1; M9362 K896 29.4 -> 26.4).  Gate/up + SwiGLU: see stream_grid.
 template <typename T, bool DUAL>

@@ -382,8 +382,11 @@ int dispatch_v2(const void* q, const void* k, const void* v, const void* mask, i
   // per CU (B3 T1000 fp16 exact with a mask 34.9 -> 27.9 us, B4 T512 18.3 ->
   // 15.7, B1 T1000 online 13.6 -> 10.5), or two where sequences are long enough
   // for the causal imbalance to matter (B1 T4096 57.7 -> 51.3, B2 T2048 exact
-  // 46.2 -> 41.8).  Deeper grids keep the whole group: B8 T512 20.4 us, split
-  // 24.4; B8 T800 37.5, split 49.2.
+  // 46.2 -> 41.8).  Deeper grids keep the whole group: B8 T800 37.5 us, split
+  // 49.2.  Between one and a half and two rounds below 1024 tokens the two sides
+  // depend on the mask (whole | split, exact): with one B8 T512 23.4 | 27.7, B12
+  // T300 18.2 | 21.8; with the causal flag B4 T1000 fp16 32.5 | 27.0.  The step at
+  // 1024 tokens is that compromise, not a change of the kernel.
   constexpr int GW = G >= 7 ? 4 : G;
   const int64_t grid16 = int64_t{kv_heads} * batch * ((tokens + 15) / 16);
   const int64_t cus = slc_host::device_cu_count();
