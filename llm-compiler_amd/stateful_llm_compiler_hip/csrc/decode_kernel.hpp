@@ -994,13 +994,13 @@ bool mfma_eligible(int dtype, int64_t head_dim, int64_t groups) {
 // which are on the device.  Graphs of back-to-back calls, us, lengths between two
 // thirds of the mask and all of it, and in brackets up to 15 % of it:
 //  * one chunk for masks up to 640 tokens, 512 at head_dim 128, and up to 1024
-//    where the grid leaves two chunks at most.  Splitting gains less there than the merge costs at
-//    head_dim 64 (L512 B16 one 7.8 [5.1], two 8.6 [7.2]; B64 L1024 12.0 [5.8],
-//    two 13.5 [9.9]).  At 128 it depends on the lengths: full caches are better
-//    split (two KV heads, B16 L512 one 11.8 [6.4], two 11.1 [8.3]; L640 13.6 [6.5],
-//    three 11.5 [8.9]; B64 L1024 20.4 [7.8], two 18.9 [11.4]), emptier ones are
-//    not: over 15, 75 and 100 % one chunk is 5 to 12 % less in sum at 512 and 1024
-//    and no less at 640;
+//    where the grid leaves two chunks at most.  Splitting gains less there than
+//    the merge costs at head_dim 64 (L512 B16 one 7.8 [5.1], two 8.6 [7.2]; B64
+//    L1024 12.0 [5.8], two 13.5 [9.9]).  At 128 it depends on the lengths: full
+//    caches are better split (two KV heads, B16 L512 one 11.8 [6.4], two 11.1
+//    [8.3]; L640 13.6 [6.5], three 11.5 [8.9]; B64 L1024 20.4 [7.8], two 18.9
+//    [11.4]), emptier ones are not: over 15, 75 and 100 % one chunk is 5 to 12 %
+//    less in sum at 512 and 1024 and no less at 640;
 //  * else equal chunks of at least 256 tokens, at most one workgroup per CU
 //    (B20 L17963 D128: six chunks of 3072 tokens 68, five of 4096 80);
 //  * chunk^2 >= 16 mask_len, which balances the chunk against the merge for few
